@@ -38,10 +38,11 @@ __global__ void k_status_init(mdd::Status* st) {
     st->abort_step = INT_MAX;
     st->error = 0;
     st->overflow = 0u;
+    st->third = 0;
     st->max_row = 0;
     st->max_half = 0;
     st->ghost_total = 0u;
-    st->overlap_count = 0;
+    st->overlap_count[0] = st->overlap_count[1] = 0;
     st->nh_kind[0] = st->nh_kind[1] = 1;
     st->hist_records = 0u;
     st->listed = 0u;
@@ -181,7 +182,12 @@ void run_steps(Ctx& c, int64_t nsteps) {
         mdd::launch_post(c, int(c.step));
         c.post_pending = false;
     }
+    // pre_done: the step whose first half the last force pass did already;
+    // fused: the passes of the running chunk that integrate, newest last
+    int pre_done = -1;
+    std::vector<int> fused;
     auto first_half = [&](int s, bool check) {
+        if (s == pre_done) return;
         if (c.post_pending) {
             mdd::launch_post_pre(c, s, check);
             c.post_pending = false;
@@ -195,10 +201,32 @@ void run_steps(Ctx& c, int64_t nsteps) {
         else
             mdd::launch_post(c, s);
     };
+    // needs_rebuild with every > 0 (neighbor.rs:605-627): steps_since_build
+    // is 0 after the build of step b and grows by one at each later step's
+    // check that keeps the list, so the count forces a rebuild at b + every + 1
+    auto count_due = [&](int64_t s) {
+        return c.every > 0 && s >= c.last_rebuild + int64_t(c.every) + 1;
+    };
+    // the force pass of step s and what follows it: on to the first half of
+    // step s + 1 in the same launch unless the run ends or the list is due
+    auto force_pass = [&](int s) {
+        if (s < end && !count_due(int64_t(s) + 1) && mdd::step_fusable(c, s)) {
+            mdd::launch_pair_forces(c, s, false, true);
+            mdd::swap_step_buffers(c);
+            fused.push_back(s);
+            pre_done = s + 1;
+            c.post_pending = false;
+        } else {
+            pre_done = -1;
+            mdd::launch_pair_forces(c, s, false);
+            second_half(s);
+        }
+    };
     // resume at the force pass of step ab after the device stopped there:
     // a rebuild request from the drift, or a rebuild that did not fit
     auto resume = [&](int ab) {
         const bool retry = (c.status_host->overflow & 31u) != 0u;
+        const int64_t prev_rebuild = c.last_rebuild;
         // the rebuild's first kernel clears the abort
         if (retry) {
             if (c.status_host->overflow & 4u) mdd::remove_outside(c);
@@ -214,48 +242,44 @@ void run_steps(Ctx& c, int64_t nsteps) {
         if (ab != c.last_resume) c.repeats = 0;
         c.last_resume = ab;
         mdd::rebuild_async(c, ab, retry);
-        mdd::launch_pair_forces(c, ab, false);
-        second_half(ab);
+        if (!retry) c.last_rebuild = ab;
+        force_pass(ab);
         if (!retry) {
             // the next chunk ends near the expected next rebuild (0.85 of
             // the interval, plus one step): launches after a rebuild request
             // return at once but still cost about 2 us each, and an early
             // end costs one more host round trip
-            const int64_t ran = int64_t(ab) - c.last_rebuild;
+            const int64_t ran = int64_t(ab) - prev_rebuild;
             if (ran > 0) {
                 c.rb_interval = c.rb_interval > 0.0 ? 0.5 * c.rb_interval + 0.5 * double(ran)
                                                     : double(ran);
                 c.chunk = int(std::min(1024.0, std::ceil(kChunkOvershoot * c.rb_interval) + 1.0));
             }
-            c.last_rebuild = ab;
         }
         c.step = ab;
     };
     auto check_status = [&]() {
         sync_status(c);
         harvest_profile(c);
+        // passes at or past the abort step did not run: their buffers go back
+        const int ab = c.status_host->abort_step;
+        for (; !fused.empty() && fused.back() >= ab; fused.pop_back()) mdd::swap_step_buffers(c);
+        fused.clear();
         check_device_error(c);
-        return c.status_host->abort_step;
-    };
-    // needs_rebuild with every > 0 (neighbor.rs:605-627): steps_since_build
-    // is 0 after the build of step b and grows by one at each later step's
-    // check that keeps the list, so the count forces a rebuild at b + every + 1
-    auto count_due = [&](int64_t s) {
-        return c.every > 0 && s >= c.last_rebuild + int64_t(c.every) + 1;
+        return ab;
     };
     for (;;) {
         while (c.step < end) {
             const int64_t s = c.step + 1;
-            const bool forced = !c.list_valid || c.list_injected || c.list_lg != c.lg ||
+            const bool forced = !c.list_valid || c.list_injected || c.list_lanes != c.lanes ||
                                 c.list_tile != c.want_tile() || count_due(s);
             if (forced) {
                 // FullRebuild step: integrate, rebuild, force, integrate
                 first_half(int(s), false);
                 mdd::rebuild_async(c, int(s), false);
-                mdd::launch_pair_forces(c, int(s), false);
-                second_half(int(s));
-                c.step = s;
                 c.last_rebuild = s;
+                force_pass(int(s));
+                c.step = s;
                 continue;
             }
             int64_t K = std::min<int64_t>(c.chunk, end - c.step);
@@ -266,8 +290,7 @@ void run_steps(Ctx& c, int64_t nsteps) {
                 first_half(st, true);
                 // sort_atoms_by_bin's periodic sort: a rebuild unless still sorted
                 if (c.sort_every > 0 && st % c.sort_every == 0) mdd::launch_sort_check(c, st);
-                mdd::launch_pair_forces(c, st, false);
-                second_half(st);
+                force_pass(st);
             }
             if (c.prof_every > 0 && c.rb_mark) {
                 MDD_HIP(hipEventRecord(c.rb_mark, c.stream));
@@ -323,6 +346,7 @@ void pack_upload(Ctx& c, int64_t n, const uint32_t* tag, const uint32_t* type, c
     c.n = n;
     c.xq_valid = false;
     c.npad = (cap + 63) / 64 * 64;
+    if (c.third) mdd::swap_state(c);
     const int64_t np = c.npad;
     c.pos.resize(np);
     c.vel.resize(np);
@@ -1223,6 +1247,7 @@ int mdd_set_half_list(mdd_ctx* ctx, int64_t nlocal, const uint32_t* offsets,
         for (int64_t i = 0; i < c.n; i++) mx = std::max<int>(mx, int(own[i].size() + rev[i].size()));
         if (c.model == MDD_MODEL_DEM && mx > 64)
             throw ApiError(MDD_ERR_UNSUPPORTED, "DEM rows above 64 entries");
+        c.lg = c.row_layout();
         const int G = 1 << c.lg;
         mx = (mx + G - 1) / G * G;
         c.maxnb = mx;
@@ -1251,6 +1276,7 @@ int mdd_set_half_list(mdd_ctx* ctx, int64_t nlocal, const uint32_t* offsets,
         c.listed_ok = false;
         c.list_tile = false;
         c.list_lg = c.lg;
+        c.list_lanes = c.lanes;
         c.npairs = offsets[c.n];
     });
 }
@@ -1641,7 +1667,10 @@ int mdd_set_force_lanes(mdd_ctx* ctx, int log2_lanes) {
             throw ApiError(MDD_ERR_INVALID, "log2 lanes per particle must be -1..3");
         // the next step rebuilds the list in the new layout
         c.tile_enabled = log2_lanes < 0;
-        if (log2_lanes >= 0) c.lg = log2_lanes;
+        if (log2_lanes >= 0) {
+            c.lanes = log2_lanes;
+            c.lanes_auto = false;
+        }
     });
 }
 

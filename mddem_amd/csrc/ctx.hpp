@@ -232,10 +232,11 @@ struct Status {
                              // bit 2: particle outside a non-periodic face,
                              // bit 3: candidate list beyond 16-bit tile indices
                              // bit 4: more old contacts than history records
+    int third;               // rebuild: the state is in the third buffers
     int max_row;             // longest full-list row at the last build
     int max_half;            // longest half-list row at the last build
     unsigned ghost_total;    // periodic images at the last build
-    int overlap_count;       // large-overlap pairs in the current step
+    int overlap_count[2];    // large-overlap pairs, by step parity
     int nh_kind[2];          // per step parity: 1 = nh_p is p_xi after a post
                              // half-update (or the initial p_xi), 0 = after a pre
     unsigned hist_records;   // contacts of the old list at the last history remap
@@ -339,6 +340,7 @@ struct Ctx {
     WallsP walls{};
     DBuf<WallsP> walls_dev;   // device copy of the wall table (integrators)
     DBuf<WallsDyn> wdyn;      // current wall points, velocities, force sums
+    DBuf<WallsDyn> wdyn2;     // those of the coming step while a pass integrates
     bool walls_moving = false;
 
     // ---- batched ensemble (nsys > 0): particles of system s are
@@ -372,8 +374,16 @@ struct Ctx {
     int64_t n = 0, cap = 0, npad = 0;
     int64_t ghost_cap = 0, nghost = 0;
     int maxnb = 0;          // row capacity of the full list (multiple of 1 << lg)
-    int lg = 2;             // log2 of lanes per particle in the pair-force kernels
-    int list_lg = 2;        // the row layout the current list was built with
+    // log2 of lanes per particle in the pair-force kernels: the caller's
+    // choice (mdd_set_force_lanes) or, for DEM until it is made, lanes_auto:
+    // the kernels then pick 1 or 2 lanes and keep the sums in the order of
+    // four, on rows laid out for two
+    int lanes = 2;
+    bool lanes_auto = true;
+    int list_lanes = 2;     // lanes when the current list was built
+    int lg = 2;             // row layout of the next list (row_layout) ...
+    int list_lg = 2;        // ... and of the current one
+    int row_layout() const { return model == 1 && lanes_auto ? 1 : lanes; }
     int lg_old = 2;         // the row layout of the previous list
     int64_t npairs = 0;
     bool list_valid = false;
@@ -404,6 +414,12 @@ struct Ctx {
     DBuf<double> f64, t64;  // 3*npad SoA force / torque (FP64 mode)
     DBuf<float> f32, t32;   // 3*npad SoA force / torque (mixed mode)
     DBuf<double4> build_pos;
+    // the other side of a force pass that integrates (allocated by the first
+    // one): swapped with pos / vel / omega at each such pass; third: pos, vel
+    // and omega are now the buffers these members started with
+    DBuf<double4> pos3, vel3, omega3;
+    bool third = false;
+    bool sorted_third = false;  // third at the last sort (its source)
     // alternates for the rebuild permutation
     DBuf<double4> pos2, vel2, omega2, quat2;
     DBuf<uint32_t> tag2, type2;
@@ -439,6 +455,7 @@ struct Ctx {
     // xq current while xq_valid and the rebuild's permutation rewrites it;
     // an upload or a box change clears it and the next pair pass refills it.
     DBuf<int4> xq;
+    DBuf<int4> xq2;        // the coming step's, written by a pass that integrates
     bool lj_fixed = true;  // mdd_set_lj_positions
     bool xq_valid = false;
     // the same fixed-point form of the build positions, written by the
@@ -464,6 +481,9 @@ struct Ctx {
     // the final half step of step `step` is deferred into the next step's
     // first pass (runs without a thermostat)
     bool post_pending = false;
+    // runs without a thermostat: the force pass of a step does that step's
+    // final half and the next step's first half as well, one launch per step
+    bool step_fused = true;
     // neighbor build kernel: 0 chosen by occupancy, 1 one wavefront per cell,
     // 2 one lane per member slot (sparse grids)
     int build_mode = 0;
@@ -580,7 +600,8 @@ void launch_sort_check(Ctx& c, int step);
 void release_graphs(Ctx& c);
 bool rebuild_grow(Ctx& c, const Status& s);
 // forces.hip
-void launch_pair_forces(Ctx& c, int step, bool energy);
+// integrate: the pass goes on to the next step's first half (step_fusable)
+void launch_pair_forces(Ctx& c, int step, bool energy, bool integrate = false);
 void launch_walls_gravity(Ctx& c, bool walls, bool gravity);
 // standalone wall_move / wall_zero_force_accumulators
 void launch_wall_systems(Ctx& c, bool move, bool zero);
@@ -600,6 +621,9 @@ inline void set_contact_path(Ctx& c, bool on) {
     }
 }
 // integrate.hip
+bool step_fusable(const Ctx& c, int step);
+void swap_step_buffers(Ctx& c);
+void swap_state(Ctx& c);
 void launch_pre(Ctx& c, int step, bool check_rebuild);
 void launch_post_pre(Ctx& c, int step, bool check_rebuild);
 void launch_post(Ctx& c, int step);

@@ -18,7 +18,7 @@
 #include <hip/hip_ext.h>
 
 #include "cells.hpp"
-#include "ctx.hpp"
+#include "step.hpp"
 
 // row entries per lane gathered together by the LJ row kernel
 #ifndef MDD_LJ_BATCH
@@ -42,6 +42,7 @@ constexpr int kXRolling = 0, kXTwisting = 1, kXCohesion = 2, kXSurface = 3, kXKn
 struct ForceArgs {
     int64_t n, npad;
     int maxnb;
+    int rl;  // row layout (row_addr) of the list
     const double4* pos;
     const double4* vel;
     const double4* omega;
@@ -89,6 +90,9 @@ struct ForceArgs {
 __device__ inline bool gated(const ForceArgs& a) {
     return a.step >= 0 && a.st->abort_step <= a.step;
 }
+
+// the step's counter of large overlaps (standalone passes: slot 0)
+__host__ __device__ inline int overlap_slot(int step) { return step >= 0 ? step & 1 : 0; }
 
 template <typename R>
 __device__ inline R rcp(R x);
@@ -211,11 +215,22 @@ __device__ inline void lj_row_fixed_force(const ForceArgs& a, int64_t i, int t, 
     fz_out = group_sum<G>(fz);
 }
 
-template <int LG>
-__device__ inline void lj_row_fixed(const ForceArgs& a, int64_t i, int t) {
+// the launch's first thread, in a pass that integrates
+template <typename S>
+__device__ inline void begin_step(const ForceArgs& a, const S& s) {
+    if constexpr (std::is_same<S, StepArgs>::value)
+        if (blockIdx.x == 0 && threadIdx.x == 0) step_begin(s, a.wdyn);
+}
+
+template <int LG, typename S>
+__device__ inline void lj_row_fixed(const ForceArgs& a, const S& s, int64_t i, int t) {
     float fx, fy, fz;
     lj_row_fixed_force<LG>(a, i, t, fx, fy, fz);
     if (t != 0) return;
+    if constexpr (std::is_same<S, StepArgs>::value) {
+        step_advance(s, i, a.pos[i], step_load(s, i), double(fx), double(fy), double(fz), 0.0, 0.0, 0.0);
+        return;
+    }
     a.f32[i] = fx;
     a.f32[a.npad + i] = fy;
     a.f32[2 * a.npad + i] = fz;
@@ -290,8 +305,8 @@ __global__ void __launch_bounds__(256 << LG) k_lj_post(ForceArgs a, PostArgs p) 
 // F_i = -fpair d'' in both cases: d = (x_j + S_j) - (x_i + S_i) with S on
 // the non-owner. Without an image both shifts vanish and d = x_j - x_i.
 // Pairs outside the cutoff contribute fma(0, d, f) = f.
-template <typename R, bool ENERGY, int LG>
-__global__ void __launch_bounds__(256) k_lj(ForceArgs a) {
+template <typename R, bool ENERGY, int LG, typename S>
+__global__ void __launch_bounds__(256) k_lj(ForceArgs a, S s) {
     constexpr int G = 1 << LG;
     // XCD-aware block order: each XCD's L2 holds the positions of one
     // contiguous (spatially sorted) range of particles and its neighbors
@@ -321,9 +336,10 @@ __global__ void __launch_bounds__(256) k_lj(ForceArgs a) {
     __syncthreads();
     if (i >= a.n) return;
     if (gated(a)) return;
+    begin_step(a, s);
     if constexpr (sizeof(R) == 4 && !ENERGY) {
         if (a.xq) {
-            lj_row_fixed<LG>(a, i, t);
+            lj_row_fixed<LG>(a, s, i, t);
             return;
         }
     }
@@ -345,16 +361,16 @@ __global__ void __launch_bounds__(256) k_lj(ForceArgs a) {
         const R r2inv = rcp<R>(R(r2));
         const R r6inv = r2inv * r2inv * r2inv;
         const R fpair = r2inv * r6inv * fma(lj1, r6inv, -lj2);
-        const R s = in ? -fpair : R(0);
-        fx = fma(s, R(dx), fx);
-        fy = fma(s, R(dy), fy);
-        fz = fma(s, R(dz), fz);
+        const R sc = in ? -fpair : R(0);
+        fx = fma(sc, R(dx), fx);
+        fy = fma(sc, R(dy), fy);
+        fz = fma(sc, R(dz), fz);
         if (ENERGY && in) {
             const double r6 = double(r6inv);
             pe += 0.5 * (r6 * (a.e12 * r6 - a.e6));
             // virial (md_lj/src/lib.rs:555-561): d (x) F per pair, half on
             // each side of the full rows (both sides see the same d (x) F)
-            const double sd = double(s);
+            const double sd = double(sc);
             w[0] += 0.5 * (dx * (sd * dx));
             w[1] += 0.5 * (dy * (sd * dy));
             w[2] += 0.5 * (dz * (sd * dz));
@@ -415,6 +431,10 @@ __global__ void __launch_bounds__(256) k_lj(ForceArgs a) {
         for (int k = 0; k < 6; k++) w[k] = group_sum<G>(w[k]);
     }
     if (t != 0) return;
+    if constexpr (std::is_same<S, StepArgs>::value) {
+        step_advance(s, i, xi, step_load(s, i), double(fx), double(fy), double(fz), 0.0, 0.0, 0.0);
+        return;
+    }
     if constexpr (sizeof(R) == 8) {
         a.f64[i] = fx;
         a.f64[a.npad + i] = fy;
@@ -960,7 +980,7 @@ __device__ inline bool pair_geom(const ForceArgs& a, const double4& pi, const do
     g.delta = sum_r - g.distance;
     if (0.5 * r_min < g.delta) g.delta = 0.5 * r_min;
     if (g.delta > 0.0 && !rev && g.distance / sum_r < kLargeOverlap) {
-        int c = atomicAdd(&a.st->overlap_count, 1) + 1;
+        int c = atomicAdd(&a.st->overlap_count[overlap_slot(a.step)], 1) + 1;
         if (c > kMaxOverlapWarnings) {
             atomicCAS(&a.st->error, 0, -3);
             if (a.step >= 0) atomicMin(&a.st->abort_step, a.step);
@@ -1125,10 +1145,26 @@ __device__ inline const SysP* particle_box(const ForceArgs& a, int64_t i, double
     return S;
 }
 
-// walls, gravity and the store of one particle's sums (lane t == 0)
-template <typename R>
-__device__ inline void finish_particle(const ForceArgs& a, int64_t i, const double4& pi, uint32_t ti,
-                                       R fx, R fy, R fz, R tx, R ty, R tz) {
+// the integration's inputs of one particle (empty without StepArgs)
+template <typename S>
+struct Pre {};
+template <>
+struct Pre<StepArgs> {
+    StepIn in;
+};
+template <typename S>
+__device__ inline Pre<S> preload(const S& s, int64_t i) {
+    Pre<S> p;
+    if constexpr (std::is_same<S, StepArgs>::value) p.in = step_load(s, i);
+    return p;
+}
+
+// walls, gravity and the store of one particle's sums (lane t == 0), or,
+// with StepArgs, its final half and next first half step with them
+template <typename R, typename S>
+__device__ inline void finish_particle(const ForceArgs& a, const S& s, int64_t i, const double4& pi,
+                                       const Pre<S>& pre, uint32_t ti, R fx, R fy, R fz, R tx, R ty,
+                                       R tz) {
     if (a.use_walls)
         wall_forces<R>(a, pi, &a.vel[i], a.omega ? &a.omega[i] : nullptr, a.mass[i], ti, fx, fy, fz,
                        tx, ty, tz);
@@ -1138,7 +1174,11 @@ __device__ inline void finish_particle(const ForceArgs& a, int64_t i, const doub
         fy += R(m * a.g[1]);
         fz += R(m * a.g[2]);
     }
-    store_force<R>(a, i, fx, fy, fz, tx, ty, tz);
+    if constexpr (std::is_same<S, StepArgs>::value)
+        step_advance(s, i, pi, pre.in, double(fx), double(fy), double(fz), double(tx),
+                     double(ty), double(tz));
+    else
+        store_force<R>(a, i, fx, fy, fz, tx, ty, tz);
 }
 
 // hertz_mindlin_contact_force (dem_granular/src/contact.rs:103-615) for
@@ -1147,15 +1187,111 @@ __device__ inline void finish_particle(const ForceArgs& a, int64_t i, const doub
 // (contact.rs:559-569): each particle sums d (x) F over the pairs it owns,
 // d = partner image - owner, F = -F_n + F_t the force on the owner, into
 // vir[q * npad + i] (xx yy zz xy xz yz).
-template <typename R, int LG, bool VIR>
-__device__ inline void hertz_particle(const ForceArgs& a, int64_t i, int t) {
+//
+// QUAD (1 or 2 lanes): the sums in the order four lanes would give, bit for
+// bit: four lanes sum the entries k = t mod 4 each, then (s0 + s2) + (s1 +
+// s3). Two lanes walk class t, then class t + 2. One lane walks its row in
+// order and changes the class it is adding to; the classes it is not adding to
+// wait in LDS (few spheres have contacts in two classes; in registers they
+// cost a wavefront per SIMD).
+template <typename R>
+struct Sums {
+    R fx = R(0), fy = R(0), fz = R(0), tx = R(0), ty = R(0), tz = R(0);
+    __device__ inline void add(const Sums& o) {
+        fx += o.fx;
+        fy += o.fy;
+        fz += o.fz;
+        tx += o.tx;
+        ty += o.ty;
+        tz += o.tz;
+    }
+};
+
+template <typename R>
+struct SumSlot {
+    R v[6][256];
+    __device__ inline void put(const Sums<R>& s) {
+        const int t = int(threadIdx.x);
+        v[0][t] = s.fx;
+        v[1][t] = s.fy;
+        v[2][t] = s.fz;
+        v[3][t] = s.tx;
+        v[4][t] = s.ty;
+        v[5][t] = s.tz;
+    }
+    __device__ inline Sums<R> get() const {
+        const int t = int(threadIdx.x);
+        Sums<R> s;
+        s.fx = v[0][t];
+        s.fy = v[1][t];
+        s.fz = v[2][t];
+        s.tx = v[3][t];
+        s.ty = v[4][t];
+        s.tz = v[5][t];
+        return s;
+    }
+};
+
+// the sums of one lane of a row: natural order, or the classes of QUAD
+template <typename R, int LG, bool QUAD>
+struct RowSums {
+    Sums<R> cur;
+    int cls = 0;
+    unsigned have = 0;  // bit c: class c has contacts
+    __device__ inline SumSlot<R>* slots() const {
+        __shared__ SumSlot<R> s[!QUAD ? 1 : (LG == 1 ? 1 : 4)];
+        return s;
+    }
+    // the next contact is entry k
+    __device__ inline void enter(int k) {
+        if (!QUAD) return;
+        const int c = k & 3;
+        if (have && c != cls) {
+            if (LG == 1) {  // class t is complete
+                slots()[0].put(cur);
+                cur = Sums<R>();
+            } else {
+                slots()[cls].put(cur);
+                cur = (have >> c) & 1u ? slots()[c].get() : Sums<R>();
+            }
+        }
+        cls = c;
+        have |= 1u << c;
+    }
+    __device__ inline Sums<R> total() const {
+        if (!QUAD || (have & (have - 1u)) == 0u) return cur;
+        if (LG == 1) {
+            Sums<R> r = slots()[0].get();
+            r.add(cur);
+            return r;
+        }
+        auto of = [&](int c) { return c == cls ? cur : slots()[c].get(); };
+        Sums<R> even, odd;
+        if (have & 1u) even = of(0);
+        if (have & 4u) even.add(of(2));
+        if (have & 2u) odd = of(1);
+        if (have & 8u) odd.add(of(3));
+        even.add(odd);
+        return even;
+    }
+};
+
+template <typename R, int LG, bool VIR, bool QUAD, typename S>
+__device__ inline void hertz_particle(const ForceArgs& a, const S& s, int64_t i, int t) {
     constexpr int G = 1 << LG;
     const double4 pi = a.pos[i];
-    R fx = R(0), fy = R(0), fz = R(0), tx = R(0), ty = R(0), tz = R(0);
-    double w0 = 0.0, w1 = 0.0, w2 = 0.0, w3 = 0.0, w4 = 0.0, w5 = 0.0;
     const uint32_t ti = a.type[i];
+    // a single system at one lane in FP32 has registers to load the
+    // integration's inputs before the row is walked (200,000 gas spheres: 18.3
+    // -> 17.5 us a step; in a batched ensemble, whose per-system lookups are
+    // the longer chain, 19.6 -> 21.4 us, so not there)
+    constexpr bool kEarly = LG == 0 && QUAD && sizeof(R) == 4;
+    Pre<S> pre;
+    if (kEarly) pre = preload(s, i);
     double Lx, Ly, Lz;
-    const SysP* S = particle_box(a, i, Lx, Ly, Lz);
+    const SysP* sys = particle_box(a, i, Lx, Ly, Lz);
+    RowSums<R, LG, QUAD> sum;
+    double w0 = 0.0, w1 = 0.0, w2 = 0.0, w3 = 0.0, w4 = 0.0, w5 = 0.0;
     if (a.use_pairs) {
         int cnt = int(a.nnb[i]);
         if (cnt > a.maxnb) cnt = a.maxnb;
@@ -1164,45 +1300,60 @@ __device__ inline void hertz_particle(const ForceArgs& a, int64_t i, int t) {
         uint64_t mask_in = 0ull;
         if (cnt > 0) mask_in = a.cmask[i];
         uint64_t mask_out = 0ull;
+        auto entry = [&](int k) {
+            return k < cnt ? a.nbr[row_addr(i, k, a.npad, a.rl)] : 0u;
+        };
+        // this lane's entry after k
+        auto after = [&](int k) {
+            if (!QUAD || LG == 0) return k + G;
+            return k + 4 < cnt || (k & 3) >= 2 ? k + 4 : (k & 3) + 2;
+        };
         // the next neighbor's position and the entry after it are loaded
         // while this one is computed (entries past the row read entry and
         // particle 0 and are not used); the partner's velocity and spin are
         // read only for pairs in contact, so they are not fetched ahead
-        uint32_t e_n = t < cnt ? a.nbr[row_addr(i, t, a.npad, LG)] : 0u;
-        uint32_t e_nn = t + G < cnt ? a.nbr[row_addr(i, t + G, a.npad, LG)] : 0u;
+        int k = t, kn = after(t);
+        uint32_t e_n = entry(k), e_nn = entry(kn);
         double4 pj_n = a.pos[entry_idx(e_n)];
-        for (int k = t; k < cnt; k += G) {
+        while (k < cnt) {
             const uint32_t e = e_n;
             const double4 pj = pj_n;
             e_n = e_nn;
             pj_n = a.pos[entry_idx(e_n)];
-            e_nn = k + 2 * G < cnt ? a.nbr[row_addr(i, k + 2 * G, a.npad, LG)] : 0u;
+            const int knn = after(kn);
+            e_nn = entry(knn);
             PairGeom g;
-            if (!pair_geom(a, pi, pj, e, Lx, Ly, Lz, g)) continue;
-            PairOut<R> o;
-            contact_pair<R>(a, S, i, ti, e, g, row_addr(i, k, a.npad, LG), (mask_in >> k) & 1ull,
-                            o);
-            if constexpr (VIR) {
-                if (!entry_rev(e)) {
-                    const double vfx = double(-o.fnx + o.ftx), vfy = double(-o.fny + o.fty),
-                                 vfz = double(-o.fnz + o.ftz);
-                    w0 += g.dx * vfx;
-                    w1 += g.dy * vfy;
-                    w2 += g.dz * vfz;
-                    w3 += g.dx * vfy;
-                    w4 += g.dx * vfz;
-                    w5 += g.dy * vfz;
+            if (pair_geom(a, pi, pj, e, Lx, Ly, Lz, g)) {
+                PairOut<R> o;
+                contact_pair<R>(a, sys, i, ti, e, g, row_addr(i, k, a.npad, a.rl),
+                                (mask_in >> k) & 1ull, o);
+                if constexpr (VIR) {
+                    if (!entry_rev(e)) {
+                        const double vfx = double(-o.fnx + o.ftx), vfy = double(-o.fny + o.fty),
+                                     vfz = double(-o.fnz + o.ftz);
+                        w0 += g.dx * vfx;
+                        w1 += g.dy * vfy;
+                        w2 += g.dz * vfz;
+                        w3 += g.dx * vfy;
+                        w4 += g.dx * vfz;
+                        w5 += g.dy * vfz;
+                    }
                 }
+                sum.enter(k);
+                add_pair<R>(entry_rev(e), o, sum.cur.fx, sum.cur.fy, sum.cur.fz, sum.cur.tx,
+                            sum.cur.ty, sum.cur.tz);
+                mask_out |= 1ull << k;
             }
-            add_pair<R>(entry_rev(e), o, fx, fy, fz, tx, ty, tz);
-            mask_out |= 1ull << k;
+            k = kn;
+            kn = knn;
         }
-        fx = group_sum<G>(fx);
-        fy = group_sum<G>(fy);
-        fz = group_sum<G>(fz);
-        tx = group_sum<G>(tx);
-        ty = group_sum<G>(ty);
-        tz = group_sum<G>(tz);
+        sum.cur = sum.total();
+        sum.cur.fx = group_sum<G>(sum.cur.fx);
+        sum.cur.fy = group_sum<G>(sum.cur.fy);
+        sum.cur.fz = group_sum<G>(sum.cur.fz);
+        sum.cur.tx = group_sum<G>(sum.cur.tx);
+        sum.cur.ty = group_sum<G>(sum.cur.ty);
+        sum.cur.tz = group_sum<G>(sum.cur.tz);
         mask_out = group_or<G>(mask_out);
         if (t == 0 && mask_out != mask_in) a.cmask[i] = mask_out;
         if constexpr (VIR) {
@@ -1224,34 +1375,26 @@ __device__ inline void hertz_particle(const ForceArgs& a, int64_t i, int t) {
         a.vir[4 * np + i] = w4;
         a.vir[5 * np + i] = w5;
     }
-    finish_particle<R>(a, i, pi, ti, fx, fy, fz, tx, ty, tz);
+    if (!kEarly) pre = preload(s, i);
+    finish_particle<R>(a, s, i, pi, pre, ti, sum.cur.fx, sum.cur.fy, sum.cur.fz, sum.cur.tx,
+                       sum.cur.ty, sum.cur.tz);
 }
 
-template <typename R, int LG, bool VIR>
-__global__ void __launch_bounds__(256) k_hertz(ForceArgs a) {
+// order: tile order (particle order[k] for k < n: each XCD works through a
+// band of bin columns, so the partners it gathers stay in its L2), or null
+// for the particles in index order
+template <typename R, int LG, bool VIR, bool QUAD, typename S>
+__global__ void __launch_bounds__(256, 3) k_hertz(ForceArgs a, S s, const uint32_t* __restrict__ order) {
     constexpr int G = 1 << LG;
     // XCD-aware block order: each XCD's L2 holds the positions of one
     // contiguous (spatially sorted) range of particles and its neighbors
-    const int64_t gt = int64_t(xcd_block(blockIdx.x, gridDim.x)) * blockDim.x + threadIdx.x;
-    const int64_t i = gt >> LG;
-    const int t = int(gt & (G - 1));
-    if (i >= a.n) return;
-    if (gated(a)) return;
-    hertz_particle<R, LG, VIR>(a, i, t);
-}
-
-// The same pass over the particles in tile order (order[k], k < n): each
-// XCD works through a band of bin columns, so the partners it gathers stay
-// in its L2; each particle's arithmetic is that of k_hertz.
-template <typename R, int LG, bool VIR>
-__global__ void __launch_bounds__(256) k_hertz_tiles(ForceArgs a, const uint32_t* __restrict__ order) {
-    constexpr int G = 1 << LG;
     const int64_t gt = int64_t(xcd_block(blockIdx.x, gridDim.x)) * blockDim.x + threadIdx.x;
     const int64_t k = gt >> LG;
     const int t = int(gt & (G - 1));
     if (k >= a.n) return;
     if (gated(a)) return;
-    hertz_particle<R, LG, VIR>(a, int64_t(order[k]), t);
+    begin_step(a, s);
+    hertz_particle<R, LG, VIR, QUAD>(a, s, order ? int64_t(order[k]) : k, t);
 }
 
 // The same pass with the pairs in contact compacted per wavefront (one lane
@@ -1339,12 +1482,14 @@ __device__ inline void wave_contacts(const ForceArgs& a, WaveQueue& q, int nq, u
 
 // order: tile order (particle order[k] for k < n), or null for XCD-aware
 // block order over the particles
-template <typename R>
-__global__ void __launch_bounds__(256) k_hertz_wave(ForceArgs a, const uint32_t* __restrict__ order) {
+template <typename R, typename S>
+__global__ void __launch_bounds__(256) k_hertz_wave(ForceArgs a, S s,
+                                                    const uint32_t* __restrict__ order) {
     __shared__ WaveQueue queues[4];
     WaveQueue& q = queues[threadIdx.x >> 6];
     const int lane = int(threadIdx.x & 63);
     if (gated(a)) return;
+    begin_step(a, s);
     const int64_t k = int64_t(xcd_block(blockIdx.x, gridDim.x)) * blockDim.x + threadIdx.x;
     const bool live = k < a.n;
     const int64_t i = live ? (order ? int64_t(order[k]) : k) : 0;
@@ -1430,7 +1575,7 @@ __global__ void __launch_bounds__(256) k_hertz_wave(ForceArgs a, const uint32_t*
         if (nq > 0) wave_contacts<R>(a, q, nq, uint32_t(i), own_lo, fx, fy, fz, tx, ty, tz);
         if (live && mask_out != mask_in) a.cmask[i] = mask_out;
     }
-    if (live) finish_particle<R>(a, i, pi, ti, fx, fy, fz, tx, ty, tz);
+    if (live) finish_particle<R>(a, s, i, pi, preload(s, i), ti, fx, fy, fz, tx, ty, tz);
 }
 
 // The same pass split by row length (one lane per particle): the particles
@@ -1439,17 +1584,18 @@ __global__ void __launch_bounds__(256) k_hertz_wave(ForceArgs a, const uint32_t*
 // state to read or write and only meets the walls and gravity, in a kernel
 // light enough to keep many wavefronts in flight. Each particle's
 // arithmetic is that of k_hertz, so the forces are the same bit for bit.
-template <typename R>
-__global__ void __launch_bounds__(256) k_hertz_listed(ForceArgs a) {
+template <typename R, typename S>
+__global__ void __launch_bounds__(256) k_hertz_listed(ForceArgs a, S s) {
     if (gated(a)) return;
+    begin_step(a, s);
     const uint32_t nl = *a.listed_n;
     const uint32_t stride = gridDim.x * blockDim.x;
     for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < nl; k += stride)
-        hertz_particle<R, 0, false>(a, int64_t(a.listed[k]), 0);
+        hertz_particle<R, 0, false, false>(a, s, int64_t(a.listed[k]), 0);
 }
 
-template <typename R>
-__global__ void __launch_bounds__(256) k_hertz_unlisted(ForceArgs a) {
+template <typename R, typename S>
+__global__ void __launch_bounds__(256) k_hertz_unlisted(ForceArgs a, S s) {
     const int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
     if (i >= a.n) return;
     if (gated(a)) return;
@@ -1473,7 +1619,11 @@ __global__ void __launch_bounds__(256) k_hertz_unlisted(ForceArgs a) {
         fy += R(m * a.g[1]);
         fz += R(m * a.g[2]);
     }
-    store_force<R>(a, i, fx, fy, fz, tx, ty, tz);
+    if constexpr (std::is_same<S, StepArgs>::value)
+        step_advance(s, i, pi, step_load(s, i), double(fx), double(fy), double(fz), double(tx),
+                     double(ty), double(tz));
+    else
+        store_force<R>(a, i, fx, fy, fz, tx, ty, tz);
 }
 
 // The contact model family on the same rows: Hertz-Mindlin with JKR / DMT
@@ -1483,8 +1633,8 @@ __global__ void __launch_bounds__(256) k_hertz_unlisted(ForceArgs a) {
 // 0-2, rolling 3-5, twist 6, canonical sign). Every pair quantity is FP64;
 // only the sums are kept in R. Pairs are evaluated in the owner frame as in
 // k_hertz, so both rows of a pair carry the same history.
-template <typename R, int LG>
-__global__ void __launch_bounds__(256) k_contact_ext(ForceArgs a) {
+template <typename R, int LG, typename S>
+__global__ void __launch_bounds__(256) k_contact_ext(ForceArgs a, S s) {
     constexpr int G = 1 << LG;
     // XCD-aware block order: each XCD's L2 holds the positions of one
     // contiguous (spatially sorted) range of particles and its neighbors
@@ -1493,6 +1643,7 @@ __global__ void __launch_bounds__(256) k_contact_ext(ForceArgs a) {
     const int t = int(gt & (G - 1));
     if (i >= a.n) return;
     if (gated(a)) return;
+    begin_step(a, s);
     const double PI = 3.141592653589793;
     const double4 pi = a.pos[i];
     const double4 vi = a.vel[i];
@@ -1511,7 +1662,7 @@ __global__ void __launch_bounds__(256) k_contact_ext(ForceArgs a) {
         const double dt = a.dt;
         const int64_t cs = a.hist_cs;
         for (int k = t; k < cnt; k += G) {
-            const int64_t slot = row_addr(i, k, a.npad, LG);
+            const int64_t slot = row_addr(i, k, a.npad, a.rl);
             const uint32_t e = a.nbr[slot];
             const uint32_t j = entry_idx(e);
             const bool rev = entry_rev(e);
@@ -1552,7 +1703,7 @@ __global__ void __launch_bounds__(256) k_contact_ext(ForceArgs a) {
             if (0.5 * r_min < delta) delta = 0.5 * r_min;
             if (a.hooke && delta <= 0.0) continue;
             if (delta > 0.0 && !rev && distance / sum_r < kLargeOverlap) {
-                int c = atomicAdd(&a.st->overlap_count, 1) + 1;
+                int c = atomicAdd(&a.st->overlap_count[overlap_slot(a.step)], 1) + 1;
                 if (c > kMaxOverlapWarnings) {
                     atomicCAS(&a.st->error, 0, -3);
                     if (a.step >= 0) atomicMin(&a.st->abort_step, a.step);
@@ -1767,16 +1918,7 @@ __global__ void __launch_bounds__(256) k_contact_ext(ForceArgs a) {
         }
     }
     if (t != 0) return;
-    if (a.use_walls)
-        wall_forces<R>(a, pi, &a.vel[i], a.omega ? &a.omega[i] : nullptr, a.mass[i], ti, fx, fy, fz, tx,
-                       ty, tz);
-    if (a.use_gravity) {
-        const double m = a.mass[i];
-        fx += R(m * a.g[0]);
-        fy += R(m * a.g[1]);
-        fz += R(m * a.g[2]);
-    }
-    store_force<R>(a, i, fx, fy, fz, tx, ty, tz);
+    finish_particle<R>(a, s, i, pi, preload(s, i), ti, fx, fy, fz, tx, ty, tz);
 }
 
 // standalone wall / gravity system: adds to the current forces
@@ -1819,13 +1961,14 @@ __global__ void k_walls_gravity(ForceArgs a) {
     f[2 * a.npad + i] = fz;
 }
 
-__global__ void k_reset_overlap(Status* st) { st->overlap_count = 0; }
+__global__ void k_reset_overlap(Status* st) { st->overlap_count[overlap_slot(-1)] = 0; }
 
 ForceArgs make_args(Ctx& c, int step) {
     ForceArgs a{};
     a.n = c.n;
     a.npad = c.npad;
     a.maxnb = c.maxnb;
+    a.rl = c.list_lg;
     a.pos = c.pos.p;
     a.vel = c.vel.p;
     a.omega = c.omega.p;
@@ -1874,21 +2017,12 @@ ForceArgs make_args(Ctx& c, int step) {
 // A pair-force launch of nb blocks of 256 threads. Timing events, when
 // given, are attached to the dispatch itself (hipExtLaunchKernelGGL), so
 // they time the kernel alone, as a kernel trace does.
-template <typename K>
-void launch_force_kernel(Ctx& c, K kern, int nb, const ForceArgs& a, hipEvent_t e0,
-                         hipEvent_t e1) {
+template <typename K, typename... A>
+void launch_force_kernel(Ctx& c, K kern, int nb, hipEvent_t e0, hipEvent_t e1, const A&... args) {
     if (e0)
-        hipExtLaunchKernelGGL(kern, dim3(nb), dim3(256), 0, c.stream, e0, e1, 0, a);
+        hipExtLaunchKernelGGL(kern, dim3(nb), dim3(256), 0, c.stream, e0, e1, 0, args...);
     else
-        kern<<<nb, 256, 0, c.stream>>>(a);
-}
-template <typename K>
-void launch_force_kernel(Ctx& c, K kern, int nb, const ForceArgs& a, hipEvent_t e0,
-                         hipEvent_t e1, const uint32_t* order) {
-    if (e0)
-        hipExtLaunchKernelGGL(kern, dim3(nb), dim3(256), 0, c.stream, e0, e1, 0, a, order);
-    else
-        kern<<<nb, 256, 0, c.stream>>>(a, order);
+        kern<<<nb, 256, 0, c.stream>>>(args...);
 }
 
 // fixed-point positions of every particle (x * qs per axis, modulo 2^32)
@@ -1919,17 +2053,16 @@ void lj_fixed_setup(Ctx& c, ForceArgs& a) {
     }
 }
 
-template <typename R, bool E>
-void launch_lj(Ctx& c, const ForceArgs& a0, hipEvent_t e0, hipEvent_t e1) {
+// a.xq is set where the pass gathers fixed-point positions (lj_fixed_setup)
+template <typename R, bool E, typename S>
+void launch_lj(Ctx& c, const ForceArgs& a, const S& s, hipEvent_t e0, hipEvent_t e1) {
     const int64_t threads = c.n << c.list_lg;
     const int nb = blocks_for(threads, 256);
-    ForceArgs a = a0;
-    if (sizeof(R) == 4 && !E && c.xq_usable()) lj_fixed_setup(c, a);
     switch (c.list_lg) {
-        case 0: launch_force_kernel(c, k_lj<R, E, 0>, nb, a, e0, e1); break;
-        case 1: launch_force_kernel(c, k_lj<R, E, 1>, nb, a, e0, e1); break;
-        case 3: launch_force_kernel(c, k_lj<R, E, 3>, nb, a, e0, e1); break;
-        default: launch_force_kernel(c, k_lj<R, E, 2>, nb, a, e0, e1); break;
+        case 0: launch_force_kernel(c, k_lj<R, E, 0, S>, nb, e0, e1, a, s); break;
+        case 1: launch_force_kernel(c, k_lj<R, E, 1, S>, nb, e0, e1, a, s); break;
+        case 3: launch_force_kernel(c, k_lj<R, E, 3, S>, nb, e0, e1, a, s); break;
+        default: launch_force_kernel(c, k_lj<R, E, 2, S>, nb, e0, e1, a, s); break;
     }
 }
 
@@ -1967,41 +2100,63 @@ bool launch_lj_post(Ctx& c, const ForceArgs& a0, hipEvent_t e0, hipEvent_t e1, i
     return true;
 }
 
-template <typename R, bool VIR>
-void launch_hertz(Ctx& c, const ForceArgs& a, hipEvent_t e0, hipEvent_t e1) {
-    const int64_t threads = c.n << c.list_lg;
-    const int nb = blocks_for(threads, 256);
+template <typename R, bool VIR, typename S>
+void launch_hertz(Ctx& c, const ForceArgs& a, const S& s, hipEvent_t e0, hipEvent_t e1) {
+    auto go = [&](int lanes_log2, auto kern, auto... more) {
+        launch_force_kernel(c, kern, blocks_for(c.n << lanes_log2, 256), e0, e1, a, s, more...);
+    };
+    const bool pick = c.lanes_auto;
+    const int lg = pick ? 2 : c.list_lanes;
     if (c.ext_on) {
-        switch (c.list_lg) {
-            case 0: launch_force_kernel(c, k_contact_ext<R, 0>, nb, a, e0, e1); break;
-            case 1: launch_force_kernel(c, k_contact_ext<R, 1>, nb, a, e0, e1); break;
-            case 3: launch_force_kernel(c, k_contact_ext<R, 3>, nb, a, e0, e1); break;
-            default: launch_force_kernel(c, k_contact_ext<R, 2>, nb, a, e0, e1); break;
+        switch (lg) {
+            case 0: go(0, k_contact_ext<R, 0, S>); break;
+            case 1: go(1, k_contact_ext<R, 1, S>); break;
+            case 3: go(3, k_contact_ext<R, 3, S>); break;
+            default: go(2, k_contact_ext<R, 2, S>); break;
         }
         return;
     }
     const bool tiles = c.tile_order && c.tile_ok && c.nsys == 0;
-    if (c.dem_wave && c.list_lg == 0 && !VIR) {
-        launch_force_kernel(c, k_hertz_wave<R>, nb, a, e0, e1,
-                            tiles ? static_cast<const uint32_t*>(c.tile_list.p) : nullptr);
+    const uint32_t* ord = tiles ? static_cast<const uint32_t*>(c.tile_list.p) : nullptr;
+    if (c.dem_wave && !pick && lg == 0 && !VIR) {
+        go(0, k_hertz_wave<R, S>, ord);
         return;
     }
-    if (tiles) {
-        const uint32_t* ord = c.tile_list.p;
-        switch (c.list_lg) {
-            case 0: launch_force_kernel(c, k_hertz_tiles<R, 0, VIR>, nb, a, e0, e1, ord); break;
-            case 1: launch_force_kernel(c, k_hertz_tiles<R, 1, VIR>, nb, a, e0, e1, ord); break;
-            case 3: launch_force_kernel(c, k_hertz_tiles<R, 3, VIR>, nb, a, e0, e1, ord); break;
-            default: launch_force_kernel(c, k_hertz_tiles<R, 2, VIR>, nb, a, e0, e1, ord); break;
+    if constexpr (!VIR) {
+        if (pick) {
+            // short rows fill the chip at one lane per sphere from about 65,000
+            // spheres on; fewer spheres, or longer rows, take two. A step of a
+            // gas at one / two lanes: 70,000 spheres 9.4 / 9.5 us, 120,000 12.4
+            // / 16.1, 200,000 17.9 / 21.0, 40,000 10.1 / 9.2, 20,000 8.6 / 7.6
+            // (four lanes: 8.2 and, at 200,000, 29.4); a bed of 250,000 72 / 68,
+            // of 20,000 29 / 23. Tile order pays on full rows only (a gas of
+            // 200,000: 17.9 us with it, 17.0 without).
+            if (c.n >= 65536 && 10 * int64_t(c.status_host->listed) < 9 * c.n)
+                go(0, k_hertz<R, 0, false, true, S>, static_cast<const uint32_t*>(nullptr));
+            else
+                go(1, k_hertz<R, 1, false, true, S>, ord);
+            return;
         }
+    }
+    switch (lg) {
+        case 0: go(0, k_hertz<R, 0, VIR, false, S>, ord); break;
+        case 1: go(1, k_hertz<R, 1, VIR, false, S>, ord); break;
+        case 3: go(3, k_hertz<R, 3, VIR, false, S>, ord); break;
+        default: go(2, k_hertz<R, 2, VIR, false, S>, ord); break;
+    }
+}
+
+// the DEM pair pass of one kernel, or split by row length
+template <typename R, typename S>
+void launch_dem(Ctx& c, const ForceArgs& a, const S& s, bool split, hipEvent_t e0, hipEvent_t e1) {
+    if (!split) {
+        launch_hertz<R, false>(c, a, s, e0, e1);
         return;
     }
-    switch (c.list_lg) {
-        case 0: launch_force_kernel(c, k_hertz<R, 0, VIR>, nb, a, e0, e1); break;
-        case 1: launch_force_kernel(c, k_hertz<R, 1, VIR>, nb, a, e0, e1); break;
-        case 3: launch_force_kernel(c, k_hertz<R, 3, VIR>, nb, a, e0, e1); break;
-        default: launch_force_kernel(c, k_hertz<R, 2, VIR>, nb, a, e0, e1); break;
-    }
+    const int nb = blocks_for(c.n, 256);
+    const int nbl = nb < 2048 ? nb : 2048;
+    k_hertz_listed<R, S><<<nbl, 256, 0, c.stream>>>(a, s);
+    k_hertz_unlisted<R, S><<<nb, 256, 0, c.stream>>>(a, s);
 }
 
 }  // namespace
@@ -2020,7 +2175,7 @@ void upload_materials(Ctx& c) {
 }
 
 // one pair-force pass (Force phase). step < 0: ungated standalone call.
-void launch_pair_forces(Ctx& c, int step, bool energy) {
+void launch_pair_forces(Ctx& c, int step, bool energy, bool integrate) {
     ForceArgs a = make_args(c, step);
     const bool mixed = c.precision == 1;
     if (step < 0) {
@@ -2049,10 +2204,12 @@ void launch_pair_forces(Ctx& c, int step, bool energy) {
     // dilute cloud): the light kernel then covers most of them. In a dense
     // packing every particle is listed and the one-kernel pass (XCD-aware
     // block order, one thread per particle) is the faster one.
-    const bool sparse_rows = c.dem_split == 1 ||
-                             (c.dem_split < 0 && 2 * int64_t(c.status_host->listed) < c.n);
+    const bool sparse_rows =
+        c.dem_split == 1 ||
+        (c.dem_split < 0 && !integrate && 2 * int64_t(c.status_host->listed) < c.n);
     const bool split = c.model == 1 && c.listed_ok && c.list_valid && !c.list_injected &&
-                       c.list_lg == 0 && !c.ext_on && c.nsys == 0 && !dem_vir && sparse_rows;
+                       !c.lanes_auto && c.list_lanes == 0 && !c.ext_on && c.nsys == 0 &&
+                       !dem_vir && sparse_rows;
     const bool one_kernel = !(c.model == 0 && c.list_tile) && !split &&
                             !(c.model == 1 && step >= 0 && c.walls.count > 0 && a.has_regions);
     if (prof) {
@@ -2079,17 +2236,25 @@ void launch_pair_forces(Ctx& c, int step, bool energy) {
             a.pe = c.pe.p;
             a.vir = c.vir.p;
             if (mixed)
-                launch_lj<float, true>(c, a, k0, k1);
+                launch_lj<float, true>(c, a, NoStep{}, k0, k1);
             else
-                launch_lj<double, true>(c, a, k0, k1);
+                launch_lj<double, true>(c, a, NoStep{}, k0, k1);
         } else if (mixed && launch_lj_post(c, a, k0, k1, step)) {
             c.last_force_fused = true;
             c.fused_rows = true;
         } else {
-            if (mixed)
-                launch_lj<float, false>(c, a, k0, k1);
-            else
-                launch_lj<double, false>(c, a, k0, k1);
+            if (mixed && c.xq_usable()) lj_fixed_setup(c, a);
+            if (integrate) {
+                const StepArgs s = step_args(c, step);
+                if (mixed)
+                    launch_lj<float, false>(c, a, s, k0, k1);
+                else
+                    launch_lj<double, false>(c, a, s, k0, k1);
+            } else if (mixed) {
+                launch_lj<float, false>(c, a, NoStep{}, k0, k1);
+            } else {
+                launch_lj<double, false>(c, a, NoStep{}, k0, k1);
+            }
         }
     } else {
         a.use_pairs = 1;
@@ -2102,24 +2267,22 @@ void launch_pair_forces(Ctx& c, int step, bool energy) {
         if (split) {
             a.listed = c.listed.p;
             a.listed_n = c.listed_n.p;
-            const int nb = blocks_for(c.n, 256);
-            const int nbl = nb < 2048 ? nb : 2048;
-            if (mixed) {
-                k_hertz_listed<float><<<nbl, 256, 0, c.stream>>>(a);
-                k_hertz_unlisted<float><<<nb, 256, 0, c.stream>>>(a);
-            } else {
-                k_hertz_listed<double><<<nbl, 256, 0, c.stream>>>(a);
-                k_hertz_unlisted<double><<<nb, 256, 0, c.stream>>>(a);
-            }
-        } else if (dem_vir) {
+        }
+        if (dem_vir) {
             if (mixed)
-                launch_hertz<float, true>(c, a, k0, k1);
+                launch_hertz<float, true>(c, a, NoStep{}, k0, k1);
             else
-                launch_hertz<double, true>(c, a, k0, k1);
+                launch_hertz<double, true>(c, a, NoStep{}, k0, k1);
+        } else if (integrate) {
+            const StepArgs s = step_args(c, step);
+            if (mixed)
+                launch_dem<float>(c, a, s, split, k0, k1);
+            else
+                launch_dem<double>(c, a, s, split, k0, k1);
         } else if (mixed) {
-            launch_hertz<float, false>(c, a, k0, k1);
+            launch_dem<float>(c, a, NoStep{}, split, k0, k1);
         } else {
-            launch_hertz<double, false>(c, a, k0, k1);
+            launch_dem<double>(c, a, NoStep{}, split, k0, k1);
         }
         if (regions) {
             ForceArgs b = a;

@@ -23,7 +23,7 @@
 #include <mutex>
 #include <string>
 
-#include "ctx.hpp"
+#include "step.hpp"
 
 namespace mdd {
 
@@ -31,77 +31,6 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kMaxPartials = kMaxKePartials;  // blocks of a thermostatted post kernel
-
-struct IntArgs {
-    int64_t n, npad;
-    double dt;
-    double4* pos;
-    double4* vel;
-    double4* omega;
-    double4* quat;
-    const double* mass;
-    const double4* build_pos;
-    const double* f64;
-    const float* f32;
-    const double* t64;
-    const float* t32;
-    int rot;         // apply rotation half-steps
-    int vv;          // apply Verlet translational half-steps
-    int check;       // evaluate the rebuild decision
-    double thr2;     // ((skin_fraction - 1) * min_skin)^2
-    BoxP box;
-    int box_exit;
-    Status* st;
-    int step;
-    double* partial;
-    int nparts;      // KE partials left by the last post kernel
-    int q_in, q_out; // thermostat slots read / written
-    double ndof, temp, q_mass;
-    const SysP* sysp;       // batched ensemble: per-system box and threshold, or null
-    const uint32_t* psys;
-    const WallsP* walls;    // walls (device copy) and their state, or null: scheduled
-    WallsDyn* wdyn;         // steps move them (PreInitialIntegration) and clear the sums
-    int4* xq;               // fixed-point copy of the positions to keep current, or null
-    double qs[3];           // its scale 2^32 / L per axis
-    const int4* bxq;        // with xq on a periodic box: fixed-point build positions, or null
-    double qu[3];           // L / 2^32 per axis
-    double thr_band;        // |d2 - thr2| up to this: the double4 build position decides
-};
-
-__device__ inline int4 quantize_pos(const IntArgs& a, const double4& p) {
-    return make_int4(quantize_axis(p.x, a.qs[0]), quantize_axis(p.y, a.qs[1]),
-                     quantize_axis(p.z, a.qs[2]), 0);
-}
-
-__device__ inline void store_xq(const IntArgs& a, int64_t i, const double4& p) {
-    a.xq[i] = quantize_pos(a, p);
-}
-
-template <typename F>
-__device__ inline void load_f(const IntArgs& a, int64_t i, double& fx, double& fy, double& fz) {
-    if constexpr (sizeof(F) == 8) {
-        fx = a.f64[i];
-        fy = a.f64[a.npad + i];
-        fz = a.f64[2 * a.npad + i];
-    } else {
-        fx = double(a.f32[i]);
-        fy = double(a.f32[a.npad + i]);
-        fz = double(a.f32[2 * a.npad + i]);
-    }
-}
-
-template <typename F>
-__device__ inline void load_t(const IntArgs& a, int64_t i, double& tx, double& ty, double& tz) {
-    if constexpr (sizeof(F) == 8) {
-        tx = a.t64[i];
-        ty = a.t64[a.npad + i];
-        tz = a.t64[2 * a.npad + i];
-    } else {
-        tx = double(a.t32[i]);
-        ty = double(a.t32[a.npad + i]);
-        tz = double(a.t32[2 * a.npad + i]);
-    }
-}
 
 // Sum over the 256 threads of a block in a fixed order; every thread gets
 // the same bits (xor butterfly inside each wavefront: both partners add the
@@ -151,83 +80,6 @@ __device__ inline double nh_term(const IntArgs& a, double ke) {
     return (a.dt / 2.0) * (2.0 * ke - a.ndof * a.temp);
 }
 
-// displacement_exceeded (neighbor.rs:564-601) + periodic box exit (651-666)
-// for position p and the position b at the last build
-__device__ inline void rebuild_check(const IntArgs& a, int64_t i, const double4& p,
-                                     const double4& b) {
-    const BoxP* box = &a.box;
-    double thr2 = a.thr2;
-    if (a.sysp) {
-        const SysP& S = a.sysp[a.psys[i]];
-        box = &S.box;
-        thr2 = S.thr2;
-    }
-    double d[3] = {p.x - b.x, p.y - b.y, p.z - b.z};
-    const double x[3] = {p.x, p.y, p.z};
-    bool out = false;
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-        if (box->periodic[k]) {
-            const double L = box->L[k], h = L * 0.5;
-            if (d[k] > h)
-                d[k] -= L;
-            else if (d[k] < -h)
-                d[k] += L;
-            if (a.box_exit && (x[k] < box->lo[k] || x[k] >= box->hi[k])) out = true;
-        }
-    }
-    if (d[0] * d[0] + d[1] * d[1] + d[2] * d[2] > thr2 || out)
-        atomicMin(&a.st->abort_step, a.step);
-}
-
-// rebuild_check from the fixed-point position and build position (every
-// axis periodic). The int32 differences are the minimum image, and each
-// coordinate is within one quantum of its double value, so d2 is within
-// thr_band of rebuild_check's d2 near the threshold; outside the band both
-// decide alike, inside it rebuild_check decides from the double4.
-__device__ inline void rebuild_check_fixed(const IntArgs& a, int64_t i, const double4& p,
-                                           const int4& bq) {
-    const int4 q = quantize_pos(a, p);
-    const double dx = double(int(uint32_t(q.x) - uint32_t(bq.x))) * a.qu[0];
-    const double dy = double(int(uint32_t(q.y) - uint32_t(bq.y))) * a.qu[1];
-    const double dz = double(int(uint32_t(q.z) - uint32_t(bq.z))) * a.qu[2];
-    const double d2 = dx * dx + dy * dy + dz * dz;
-    if (fabs(d2 - a.thr2) <= a.thr_band) {
-        rebuild_check(a, i, p, a.build_pos[i]);
-        return;
-    }
-    bool out = false;
-    if (a.box_exit) {
-        const double x[3] = {p.x, p.y, p.z};
-#pragma unroll
-        for (int k = 0; k < 3; k++)
-            if (x[k] < a.box.lo[k] || x[k] >= a.box.hi[k]) out = true;
-    }
-    if (d2 > a.thr2 || out) atomicMin(&a.st->abort_step, a.step);
-}
-
-// orientation update of initial_rotation with the kicked omega w
-// (rotational.rs:70-83)
-__device__ inline void rotate_quat(const IntArgs& a, int64_t i, const double4& w) {
-    const double dt = a.dt;
-    const double omega_mag = sqrt(w.x * w.x + w.y * w.y + w.z * w.z);
-    const double angle = omega_mag * dt;
-    if (angle > 1e-14) {
-        const double inv = 1.0 / omega_mag;
-        const double ax = w.x * inv, ay = w.y * inv, az = w.z * inv;
-        const double half = angle * 0.5;
-        const double s = sin(half);
-        const double a0 = cos(half), a1 = ax * s, a2 = ay * s, a3 = az * s;
-        const double4 b = a.quat[i];
-        double4 q;
-        q.x = a0 * b.x - a1 * b.y - a2 * b.z - a3 * b.w;
-        q.y = a0 * b.y + a1 * b.x + a2 * b.w - a3 * b.z;
-        q.z = a0 * b.z - a1 * b.w + a2 * b.x + a3 * b.y;
-        q.w = a0 * b.w + a1 * b.z - a2 * b.y + a3 * b.x;
-        a.quat[i] = q;
-    }
-}
-
 // initial_rotation body (rotational.rs:59-84)
 __device__ inline void rotate_initial(const IntArgs& a, int64_t i, double tx, double ty,
                                       double tz) {
@@ -254,18 +106,6 @@ __device__ inline void rotate_final(const IntArgs& a, int64_t i, double tx, doub
     w.y += 0.5 * dt * ty * ii;
     w.z += 0.5 * dt * tz * ii;
     if (tx != 0.0 || ty != 0.0 || tz != 0.0) a.omega[i] = w;
-}
-
-__device__ inline void kick_drift(const IntArgs& a, double4& v, double4& p, double fx, double fy,
-                                  double fz) {
-    const double dt = a.dt;
-    const double h = 0.5 * dt * v.w;
-    v.x += h * fx;
-    v.y += h * fy;
-    v.z += h * fz;
-    p.x += v.x * dt;
-    p.y += v.y * dt;
-    p.z += v.z * dt;
 }
 
 // PreInitialIntegration + InitialIntegration of one step: thermostat
@@ -299,7 +139,7 @@ __global__ void __launch_bounds__(kThreads) k_pre(IntArgs a) {
     // uniform over the launch: only earlier kernels lower abort_step below step
     if (a.step >= 0 && a.st->abort_step < a.step) return;
     if (i == 0) {
-        a.st->overlap_count = 0;
+        a.st->overlap_count[a.step & 1] = 0;
         if (a.wdyn && a.step >= 0) walls_advance(*a.walls, *a.wdyn, a.dt);
     }
     double scale = 1.0;
@@ -395,7 +235,7 @@ __global__ void __launch_bounds__(kThreads) k_post_pre(IntArgs a) {
     const int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
     if (a.step >= 0 && a.st->abort_step < a.step) return;
     if (i == 0) {
-        a.st->overlap_count = 0;
+        a.st->overlap_count[a.step & 1] = 0;
         if (a.wdyn && a.step >= 0) walls_advance(*a.walls, *a.wdyn, a.dt);
     }
     if (i >= a.n) return;
@@ -564,7 +404,9 @@ int post_blocks(const Ctx& c, bool nh) {
     return nh ? std::min(nb, kMaxPartials) : nb;
 }
 
-IntArgs make_args(Ctx& c, int step, bool check) {
+}  // namespace
+
+IntArgs integrate_args(Ctx& c, int step, bool check) {
     IntArgs a{};
     if (c.walls.count > 0 && c.wdyn.p) {
         a.walls = c.walls_dev.p;
@@ -633,6 +475,8 @@ IntArgs make_args(Ctx& c, int step, bool check) {
     return a;
 }
 
+namespace {
+
 template <bool NH>
 void pre_impl(Ctx& c, IntArgs& a) {
     const int nb = blocks_for(c.n, kThreads);
@@ -657,7 +501,7 @@ void post_impl(Ctx& c, IntArgs& a) {
 
 // scheduled pre kernel of a step (all enabled integrators)
 void launch_pre(Ctx& c, int step, bool check_rebuild) {
-    IntArgs a = make_args(c, step, check_rebuild);
+    IntArgs a = integrate_args(c, step, check_rebuild);
     a.rot = c.rot_on && c.model == 1;
     a.vv = c.vv_on;
     if (c.nh_on)
@@ -669,7 +513,7 @@ void launch_pre(Ctx& c, int step, bool check_rebuild) {
 // the deferred final half step of step - 1 with the first half of `step`
 // (runs without a thermostat)
 void launch_post_pre(Ctx& c, int step, bool check_rebuild) {
-    IntArgs a = make_args(c, step, check_rebuild);
+    IntArgs a = integrate_args(c, step, check_rebuild);
     a.rot = c.rot_on && c.model == 1;
     a.vv = c.vv_on;
     const int nb = blocks_for(c.n, kThreads);
@@ -680,6 +524,59 @@ void launch_post_pre(Ctx& c, int step, bool check_rebuild) {
     MDD_HIP(hipGetLastError());
 }
 
+// A run without a thermostat: the force pass of a step can go on to the
+// step's final half and the next step's first half, particle by particle,
+// when nothing else has to happen between them: no wall that moves (its
+// motion may depend on the whole pass' force sum), no region walls (a pass of
+// their own after the pair pass), no contact virial of this step (its kernel
+// stores the forces) and no cell tiles.
+bool step_fusable(const Ctx& c, int step) {
+    if (!c.step_fused || c.nh_on || !c.vv_on || c.walls_moving || c.list_tile ||
+        c.list_injected || !c.list_valid)
+        return false;
+    for (int k = 0; k < c.walls.count; k++)
+        if (c.walls.w[k].kind == 3) return false;
+    return !(c.model == 1 && c.nsys == 0 && c.virial_every > 0 && step % c.virial_every == 0);
+}
+
+StepArgs step_args(Ctx& c, int step) {
+    StepArgs s{};
+    s.in = integrate_args(c, step + 1, true);
+    s.in.vv = c.vv_on;
+    s.in.rot = c.rot_on && c.model == 1;
+    c.pos3.resize(size_t(c.npad));
+    c.vel3.resize(size_t(c.npad));
+    s.pos = c.pos3.p;
+    s.vel = c.vel3.p;
+    if (c.model == 1) {
+        c.omega3.resize(size_t(c.npad));
+        s.omega = c.omega3.p;
+    }
+    if (s.in.xq) {
+        c.xq2.resize(size_t(c.npad));
+        s.in.xq = c.xq2.p;
+    }
+    if (s.in.wdyn) {
+        c.wdyn2.resize(1);
+        s.wdyn = c.wdyn2.p;
+    }
+    return s;
+}
+
+// exchange the particle state with the third buffers
+void swap_state(Ctx& c) {
+    c.pos.swap(c.pos3);
+    c.vel.swap(c.vel3);
+    if (c.model == 1) c.omega.swap(c.omega3);
+    if (c.xq2.p) c.xq.swap(c.xq2);
+    c.third = !c.third;
+}
+
+void swap_step_buffers(Ctx& c) {
+    swap_state(c);
+    if (c.wdyn2.p) c.wdyn.swap(c.wdyn2);
+}
+
 // scheduled post kernel of a step; its thermostat half uses slot step & 1
 void launch_post(Ctx& c, int step) {
     if (c.last_force_fused) {
@@ -688,7 +585,7 @@ void launch_post(Ctx& c, int step) {
         if (c.nh_on && !c.fused_rows) launch_ke_reduce(c, step, c.fused_parts);
         return;
     }
-    IntArgs a = make_args(c, step, false);
+    IntArgs a = integrate_args(c, step, false);
     a.partial = c.partial.p;
     a.rot = c.rot_on && c.model == 1;
     a.vv = c.vv_on;
@@ -701,32 +598,32 @@ void launch_post(Ctx& c, int step) {
 }
 
 void launch_initial_integration(Ctx& c, int step, bool check_rebuild) {
-    IntArgs a = make_args(c, step, check_rebuild);
+    IntArgs a = integrate_args(c, step, check_rebuild);
     a.vv = 1;
     pre_impl<false>(c, a);
 }
 
 void launch_final_integration(Ctx& c) {
-    IntArgs a = make_args(c, -1, false);
+    IntArgs a = integrate_args(c, -1, false);
     a.vv = 1;
     post_impl<false>(c, a);
 }
 
 void launch_initial_rotation(Ctx& c) {
-    IntArgs a = make_args(c, -1, false);
+    IntArgs a = integrate_args(c, -1, false);
     a.rot = 1;
     pre_impl<false>(c, a);
 }
 
 void launch_final_rotation(Ctx& c) {
-    IntArgs a = make_args(c, -1, false);
+    IntArgs a = integrate_args(c, -1, false);
     a.rot = 1;
     post_impl<false>(c, a);
 }
 
 // KE partials of the current velocities (thermostat start)
 void launch_ke_partials(Ctx& c) {
-    IntArgs a = make_args(c, -1, false);
+    IntArgs a = integrate_args(c, -1, false);
     a.partial = c.partial.p;
     k_ke_partials<<<post_blocks(c, true), kThreads, 0, c.stream>>>(a);
     MDD_HIP(hipGetLastError());
@@ -734,13 +631,13 @@ void launch_ke_partials(Ctx& c) {
 }
 
 void launch_nh_seed(Ctx& c, int parity) {
-    IntArgs a = make_args(c, -1, false);
+    IntArgs a = integrate_args(c, -1, false);
     k_nh_seed<<<1, 1, 0, c.stream>>>(a, parity & 1, 1);
     MDD_HIP(hipGetLastError());
 }
 
 void launch_nh_finish(Ctx& c, int parity) {
-    IntArgs a = make_args(c, -1, false);
+    IntArgs a = integrate_args(c, -1, false);
     k_nh_finish<<<1, kThreads, 0, c.stream>>>(a, parity & 1);
     MDD_HIP(hipGetLastError());
 }
@@ -749,7 +646,7 @@ void launch_nh_finish(Ctx& c, int parity) {
 void launch_nh_pre_standalone(Ctx& c) {
     launch_ke_partials(c);
     launch_nh_seed(c, 0);
-    IntArgs a = make_args(c, -1, false);
+    IntArgs a = integrate_args(c, -1, false);
     a.q_in = 0;
     a.q_out = 1;
     pre_impl<true>(c, a);
@@ -759,7 +656,7 @@ void launch_nh_pre_standalone(Ctx& c) {
 
 // standalone nh_post_final: scale from Status::p_xi, then the KE update
 void launch_nh_post_standalone(Ctx& c) {
-    IntArgs a = make_args(c, -1, false);
+    IntArgs a = integrate_args(c, -1, false);
     k_nh_seed<<<1, 1, 0, c.stream>>>(a, 0, 0);
     MDD_HIP(hipGetLastError());
     a.q_in = 0;

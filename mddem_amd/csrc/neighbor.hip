@@ -42,12 +42,16 @@ __device__ inline uint32_t cell_of(const GridP& g, double x, double y, double z)
 }
 
 // Start of a rebuild: the step sequence resumes (abort cleared), the build
-// status is reset and the sort's per-cell counts are zeroed.
-__global__ void k_rebuild_begin(Status* st, uint32_t* __restrict__ cnt, int64_t ncells) {
+// status is reset and the sort's per-cell counts are zeroed. third: which
+// buffers hold the state to sort (a word that the sort's kernels read, so that
+// their arguments, and with them a captured launch sequence, do not depend on it).
+__global__ void k_rebuild_begin(Status* st, uint32_t* __restrict__ cnt, int64_t ncells,
+                                int third) {
     for (int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; i < ncells;
          i += int64_t(gridDim.x) * blockDim.x)
         cnt[i] = 0u;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
+        st->third = third;
         st->abort_step = INT_MAX;
         st->overflow = 0u;
         st->max_row = 0;
@@ -61,12 +65,13 @@ __global__ void k_rebuild_begin(Status* st, uint32_t* __restrict__ cnt, int64_t 
 // of a wavefront are counted by one atomic). Batched ensembles pass the
 // per-system table: each particle then uses its own system's box and grid,
 // and its key is offset into the shared cell space.
-__global__ void k_wrap_key(int64_t n, double4* __restrict__ pos, int4* __restrict__ image,
+__global__ void k_wrap_key(int64_t n, double4* pos, double4* pos3, int4* __restrict__ image,
                            BoxP box, GridP g, uint32_t* __restrict__ key, Status* st,
                            const SysP* __restrict__ sysp, const uint32_t* __restrict__ psys,
                            uint32_t* __restrict__ cnt) {
     const int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
     const bool valid = i < n;
+    if (st->third) pos = pos3;
     uint32_t kc = 0u;
     if (valid) {
         int64_t coff = 0;
@@ -112,6 +117,8 @@ struct PermArgs {
     int64_t n, npad;
     const uint32_t* order;
     const double4 *pos, *vel, *omega, *quat;
+    const double4 *pos3, *vel3, *omega3;  // their sources when st->third
+    const Status* st;
     double4 *pos2, *vel2, *omega2, *quat2, *build_pos;
     const uint32_t *tag, *type, *key;
     uint32_t *tag2, *type2, *key2;
@@ -134,6 +141,11 @@ struct PermArgs {
 __global__ void k_permute(PermArgs a) {
     int64_t k = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
     if (k >= a.n) return;
+    if (a.st->third) {
+        a.pos = a.pos3;
+        a.vel = a.vel3;
+        a.omega = a.omega3;
+    }
     uint32_t o = a.order[k];
     double4 p = a.pos[o];
     a.pos2[k] = p;
@@ -1177,9 +1189,17 @@ void permute_all(Ctx& c, const uint32_t* order, int64_t n) {
     a.n = n;
     a.npad = c.npad;
     a.order = order;
+    // the source's arguments are the same whichever buffers hold the state:
+    // c.third tells the kernel (Status::third)
+    c.sorted_third = c.third;
+    if (c.third) swap_state(c);
     a.pos = c.pos.p;
     a.vel = c.vel.p;
     a.omega = c.omega.p;
+    a.pos3 = c.pos3.p;
+    a.vel3 = c.vel3.p;
+    a.omega3 = c.omega3.p;
+    a.st = c.status.p;
     a.quat = c.quat.p;
     a.pos2 = c.pos2.p;
     a.vel2 = c.vel2.p;
@@ -1274,12 +1294,13 @@ void rebuild_prepare(Ctx& c) {
     // reallocated while kernels that use it are queued
     c.scan_tmp.resize(size_t((std::max<int64_t>(ncells, n) + 2047) / 2048 + 2));
 
-    launch(c, k_rebuild_begin, blocks_for(ncells, 256) < 512 ? blocks_for(ncells, 256) : 512, 256,
-           c.status.p, c.cnt.p, ncells);
+    // (launched by itself: its arguments differ from rebuild to rebuild)
+    k_rebuild_begin<<<blocks_for(ncells, 256) < 512 ? blocks_for(ncells, 256) : 512, 256, 0,
+                      c.stream>>>(c.status.p, c.cnt.p, ncells, c.third ? 1 : 0);
     // pbc + keys
-    launch(c, k_wrap_key, blocks_for(n, 256), 256, n, c.pos.p, c.image.p, c.box, c.grid,
-                                                          c.key.p, c.status.p, c.sysp_or_null(),
-                                                          c.psys.p, c.cnt.p);
+    launch(c, k_wrap_key, blocks_for(n, 256), 256, n, c.third ? c.pos3.p : c.pos.p,
+           c.third ? c.pos.p : c.pos3.p, c.image.p, c.box, c.grid, c.key.p, c.status.p,
+           c.sysp_or_null(), c.psys.p, c.cnt.p);
     // sort_atoms_by_bin: stable counting sort of particles by bin
     counting_sort(c, c.key.p, n, nullptr, ncells, c.cnt.p, c.start.p, c.placed.p, c.order.p,
                   nullptr, true, nullptr, nullptr, true);
@@ -1319,6 +1340,7 @@ void rebuild_attempt(Ctx& c) {
     const bool sparse = c.nsys == 0 && !c.want_tile() &&
                         (c.build_mode == 2 || (c.build_mode == 0 && n < ncells));
     if (sparse) c.bin_cell.resize(nall_max);
+    c.lg = c.row_layout();
     const int G = 1 << c.lg;
     if (c.maxnb < G) c.maxnb = G;
     c.maxnb = (c.maxnb + G - 1) / G * G;
@@ -1504,6 +1526,7 @@ void rebuild_attempt(Ctx& c) {
     c.list_valid = true;
     c.list_injected = false;
     c.list_lg = c.lg;
+    c.list_lanes = c.lanes;
     c.npairs = -1;  // computed on request
 }
 
@@ -1585,6 +1608,7 @@ void remove_outside(Ctx& c) {
     for (int64_t j = 0; j < len; j++) fin[fill[key_pre[cur[j]]]++] = cur[j];
     // the pre-sort arrays back in place, then the survivors gathered
     swap_alternates(c);
+    if (c.sorted_third) swap_state(c);
     h2d(c, c.order.p, fin.data(), sizeof(uint32_t) * size_t(len));
     h2d(c, c.start.p, start.data(), sizeof(uint32_t) * (size_t(ncells) + 1));
     permute_all(c, c.order.p, len);
