@@ -18,10 +18,11 @@
 #include <cstring>
 #include <new>
 
-#include "ctx.hpp"
 #include "mddem_hip.h"
+#include "transfer.hpp"
 
 using mdd::ApiError;
+using mdd::ColumnKind;
 using mdd::Ctx;
 
 struct mdd_ctx {
@@ -570,6 +571,7 @@ int mdd_destroy(mdd_ctx* ctx) {
     for (hipEvent_t e : c.rb_ev) (void)hipEventDestroy(e);
     if (c.rb_mark) (void)hipEventDestroy(c.rb_mark);
     mdd::release_graphs(c);
+    mdd::release_staging(c);
     if (c.status_host) (void)hipHostFree(c.status_host);
     c.status_host = nullptr;
     hipStream_t s = c.stream;
@@ -1068,24 +1070,12 @@ int mdd_download_properties(mdd_ctx* ctx, uint32_t* type, double* mass, double* 
                             double* cutoff_radius) {
     return guarded(ctx, [&](Ctx& c) {
         need_state(c);
-        MDD_HIP(hipStreamSynchronize(c.stream));
-        const int64_t n = c.n;
-        if (type) {
-            auto h = dl(c, c.type, n);
-            std::copy(h.begin(), h.end(), type);
-        }
-        if (mass) {
-            auto h = dl(c, c.mass, n);
-            std::copy(h.begin(), h.end(), mass);
-        }
-        if (cutoff_radius) {
-            auto h = dl(c, c.cutr, n);
-            std::copy(h.begin(), h.end(), cutoff_radius);
-        }
-        if (radius) {
-            auto h = dl(c, c.pos, n);
-            for (int64_t i = 0; i < n; i++) radius[i] = h[i].w;
-        }
+        std::vector<mdd::Column> cols;
+        if (type) cols.push_back({ColumnKind::u32, c.type.p, type});
+        if (mass) cols.push_back({ColumnKind::f64, c.mass.p, mass});
+        if (cutoff_radius) cols.push_back({ColumnKind::f64, c.cutr.p, cutoff_radius});
+        if (radius) cols.push_back({ColumnKind::w, c.pos.p, radius});
+        mdd::download(c, cols.data(), int(cols.size()), c.n);
     });
 }
 
@@ -1093,80 +1083,32 @@ int mdd_download_state(mdd_ctx* ctx, uint32_t* tag, double* pos, double* vel, do
                        double* quat, int32_t* image) {
     return guarded(ctx, [&](Ctx& c) {
         need_state(c);
-        MDD_HIP(hipStreamSynchronize(c.stream));
-        const int64_t n = c.n;
-        if (tag) {
-            auto t = dl(c, c.tag, n);
-            std::copy(t.begin(), t.end(), tag);
-        }
-        if (pos) {
-            auto h = dl(c, c.pos, n);
-            for (int64_t i = 0; i < n; i++) {
-                pos[3 * i] = h[i].x;
-                pos[3 * i + 1] = h[i].y;
-                pos[3 * i + 2] = h[i].z;
-            }
-        }
-        if (vel) {
-            auto h = dl(c, c.vel, n);
-            for (int64_t i = 0; i < n; i++) {
-                vel[3 * i] = h[i].x;
-                vel[3 * i + 1] = h[i].y;
-                vel[3 * i + 2] = h[i].z;
-            }
-        }
-        if (omega) {
-            if (c.model != MDD_MODEL_DEM) throw ApiError(MDD_ERR_INVALID, "no angular state");
-            auto h = dl(c, c.omega, n);
-            for (int64_t i = 0; i < n; i++) {
-                omega[3 * i] = h[i].x;
-                omega[3 * i + 1] = h[i].y;
-                omega[3 * i + 2] = h[i].z;
-            }
-        }
-        if (quat) {
-            if (c.model != MDD_MODEL_DEM) throw ApiError(MDD_ERR_INVALID, "no orientation state");
-            auto h = dl(c, c.quat, n);
-            for (int64_t i = 0; i < n; i++) {
-                quat[4 * i] = h[i].x;
-                quat[4 * i + 1] = h[i].y;
-                quat[4 * i + 2] = h[i].z;
-                quat[4 * i + 3] = h[i].w;
-            }
-        }
-        if (image) {
-            auto h = dl(c, c.image, n);
-            for (int64_t i = 0; i < n; i++) {
-                image[3 * i] = h[i].x;
-                image[3 * i + 1] = h[i].y;
-                image[3 * i + 2] = h[i].z;
-            }
-        }
+        if (omega && c.model != MDD_MODEL_DEM) throw ApiError(MDD_ERR_INVALID, "no angular state");
+        if (quat && c.model != MDD_MODEL_DEM)
+            throw ApiError(MDD_ERR_INVALID, "no orientation state");
+        std::vector<mdd::Column> cols;
+        if (tag) cols.push_back({ColumnKind::u32, c.tag.p, tag});
+        if (pos) cols.push_back({ColumnKind::xyz, c.pos.p, pos});
+        if (vel) cols.push_back({ColumnKind::xyz, c.vel.p, vel});
+        if (omega) cols.push_back({ColumnKind::xyz, c.omega.p, omega});
+        if (quat) cols.push_back({ColumnKind::xyzw, c.quat.p, quat});
+        if (image) cols.push_back({ColumnKind::ixyz, c.image.p, image});
+        mdd::download(c, cols.data(), int(cols.size()), c.n);
     });
 }
 
 int mdd_download_forces(mdd_ctx* ctx, double* force, double* torque) {
     return guarded(ctx, [&](Ctx& c) {
         need_state(c);
-        MDD_HIP(hipStreamSynchronize(c.stream));
-        const int64_t n = c.n, np = c.npad;
+        if (torque && c.model != MDD_MODEL_DEM) throw ApiError(MDD_ERR_INVALID, "no torque state");
         const bool mixed = c.precision == MDD_MIXED;
-        auto take = [&](double* out, bool tq) {
-            if (!out) return;
-            if (tq && c.model != MDD_MODEL_DEM)
-                throw ApiError(MDD_ERR_INVALID, "no torque state");
-            if (mixed) {
-                auto h = dl(c, tq ? c.t32 : c.f32, size_t(3 * np));
-                for (int64_t i = 0; i < n; i++)
-                    for (int d = 0; d < 3; d++) out[3 * i + d] = double(h[d * np + i]);
-            } else {
-                auto h = dl(c, tq ? c.t64 : c.f64, size_t(3 * np));
-                for (int64_t i = 0; i < n; i++)
-                    for (int d = 0; d < 3; d++) out[3 * i + d] = h[d * np + i];
-            }
-        };
-        take(force, false);
-        take(torque, true);
+        const ColumnKind kind = mixed ? ColumnKind::soa32 : ColumnKind::soa64;
+        const void* f = mixed ? static_cast<const void*>(c.f32.p) : c.f64.p;
+        const void* t = mixed ? static_cast<const void*>(c.t32.p) : c.t64.p;
+        std::vector<mdd::Column> cols;
+        if (force) cols.push_back({kind, f, force});
+        if (torque) cols.push_back({kind, t, torque});
+        mdd::download(c, cols.data(), int(cols.size()), c.n);
     });
 }
 

@@ -552,6 +552,11 @@ struct Ctx {
     int64_t last_resume = -1;  // step of the last rebuild inside a run and
     int repeats = 0;           // how many times in a row it was that step
 
+    // ---- pinned staging memory of downloads, one event per slot
+    char* stage = nullptr;
+    size_t stage_bytes = 0;
+    std::vector<hipEvent_t> stage_ev;
+
     // ---- rebuild launch sequences captured as graphs
     LaunchLog rec;
     int row_nblk = 0;  // per-block row-maxima slots of the last build

@@ -1,0 +1,183 @@
+// Particle columns from the device into the caller's arrays.
+//
+// A download was a pageable copy of each device array in its padded device
+// layout (double4, int4, component-major forces) into a temporary vector, then
+// a loop that picked the components: three passes over memory that is
+// page-faulted twice, on one thread (4,000,000 spheres: 175 ms for 480 MB).
+// Here a kernel writes the caller's layout straight into pinned host memory,
+// so only the wanted bytes cross the bus, and the host copies each piece once
+// to its place. The host copy with the page faults of a fresh array is the
+// slower side (a few GB/s on one thread), so large downloads use several
+// threads, each on its own pieces.
+#include <algorithm>
+#include <atomic>
+#include <cstring>
+#include <exception>
+#include <mutex>
+#include <thread>
+
+#include "transfer.hpp"
+
+namespace mdd {
+
+namespace {
+
+// out[w], w < words: word w of particles first .. in the caller's layout
+__global__ void k_pack(ColumnKind kind, const void* __restrict__ src, int64_t npad, int64_t first,
+                       int64_t words, void* __restrict__ out) {
+    const int64_t w = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
+    if (w >= words) return;
+    const int64_t p = first + w / 3;
+    const int d = int(w % 3);
+    switch (kind) {
+        case ColumnKind::u32: static_cast<uint32_t*>(out)[w] = static_cast<const uint32_t*>(src)[first + w]; break;
+        case ColumnKind::f64: static_cast<double*>(out)[w] = static_cast<const double*>(src)[first + w]; break;
+        case ColumnKind::xyz: static_cast<double*>(out)[w] = static_cast<const double*>(src)[4 * p + d]; break;
+        case ColumnKind::w: static_cast<double*>(out)[w] = static_cast<const double*>(src)[4 * (first + w) + 3]; break;
+        case ColumnKind::xyzw: static_cast<double*>(out)[w] = static_cast<const double*>(src)[4 * first + w]; break;
+        case ColumnKind::ixyz: static_cast<int32_t*>(out)[w] = static_cast<const int32_t*>(src)[4 * p + d]; break;
+        case ColumnKind::soa32: static_cast<double*>(out)[w] = double(static_cast<const float*>(src)[d * npad + p]); break;
+        case ColumnKind::soa64: static_cast<double*>(out)[w] = static_cast<const double*>(src)[d * npad + p]; break;
+    }
+}
+
+int words_of(ColumnKind k) {
+    switch (k) {
+        case ColumnKind::xyz:
+        case ColumnKind::ixyz:
+        case ColumnKind::soa32:
+        case ColumnKind::soa64: return 3;
+        case ColumnKind::xyzw: return 4;
+        default: return 1;
+    }
+}
+size_t word_bytes(ColumnKind k) { return k == ColumnKind::u32 || k == ColumnKind::ixyz ? 4 : 8; }
+size_t row_bytes(ColumnKind k) { return size_t(words_of(k)) * word_bytes(k); }
+
+struct Piece {
+    const Column* col;
+    int64_t first, count;
+};
+
+void pack(Ctx& c, const Piece& p, void* out) {
+    const int64_t words = p.count * words_of(p.col->kind);
+    k_pack<<<blocks_for(words, 256), 256, 0, c.stream>>>(p.col->kind, p.col->dev, c.npad, p.first,
+                                                       words, out);
+    MDD_HIP(hipGetLastError());
+}
+
+void place(const Piece& p, const void* from) {
+    const size_t rb = row_bytes(p.col->kind);
+    std::memcpy(static_cast<char*>(p.col->host) + size_t(p.first) * rb, from, size_t(p.count) * rb);
+}
+
+constexpr size_t kSlot = size_t(1) << 19;  // bytes of one piece
+constexpr int kMaxCopiers = 8;             // host threads of one download
+
+// pinned staging memory of at least `bytes`, kept with the context
+char* staging(Ctx& c, size_t bytes) {
+    if (c.stage_bytes < bytes) {
+        if (c.stage) MDD_HIP(hipHostFree(c.stage));
+        c.stage = nullptr;
+        c.stage_bytes = 0;
+        MDD_HIP(hipHostMalloc(reinterpret_cast<void**>(&c.stage), bytes, hipHostMallocDefault));
+        c.stage_bytes = bytes;
+    }
+    return c.stage;
+}
+
+}  // namespace
+
+void release_staging(Ctx& c) {
+    for (hipEvent_t e : c.stage_ev) (void)hipEventDestroy(e);
+    c.stage_ev.clear();
+    if (c.stage) (void)hipHostFree(c.stage);
+    c.stage = nullptr;
+    c.stage_bytes = 0;
+}
+
+void download(Ctx& c, const Column* cols, int ncols, int64_t n) {
+    size_t total = 0;
+    for (int k = 0; k < ncols; k++) total += row_bytes(cols[k].kind) * size_t(n);
+    if (total == 0) return;
+    // up to 2 MiB (tens of thousands of particles): every column packed, one
+    // wait, one thread
+    if (total <= (size_t(2) << 20)) {
+        char* s = staging(c, total);
+        size_t at = 0;
+        // (8-byte words first, so that every column is aligned)
+        std::vector<std::pair<Piece, size_t>> ps;
+        for (const size_t wb : {size_t(8), size_t(4)})
+            for (int k = 0; k < ncols; k++) {
+                if (word_bytes(cols[k].kind) != wb) continue;
+                const Piece p{&cols[k], 0, n};
+                pack(c, p, s + at);
+                ps.emplace_back(p, at);
+                at += row_bytes(cols[k].kind) * size_t(n);
+            }
+        MDD_HIP(hipStreamSynchronize(c.stream));
+        for (const auto& p : ps) place(p.first, s + p.second);
+        return;
+    }
+    std::vector<Piece> pieces;
+    for (int k = 0; k < ncols; k++) {
+        const int64_t per = int64_t(kSlot / row_bytes(cols[k].kind));
+        for (int64_t f = 0; f < n; f += per)
+            pieces.push_back({&cols[k], f, std::min(per, n - f)});
+    }
+    const int np = int(pieces.size());
+    const int cpus = int(std::thread::hardware_concurrency());
+    const int copiers = std::max(1, std::min({kMaxCopiers, np / 2, cpus > 1 ? cpus / 2 : 1}));
+    const int slots = std::min(np, 2 * copiers);
+    char* s = staging(c, size_t(slots) * kSlot);
+    while (int(c.stage_ev.size()) < slots) {
+        hipEvent_t e;
+        MDD_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        c.stage_ev.push_back(e);
+    }
+    // piece q goes through slot q mod slots: packed, then placed, then the
+    // slot takes piece q + slots
+    auto issue = [&](int q) {
+        pack(c, pieces[size_t(q)], s + size_t(q % slots) * kSlot);
+        MDD_HIP(hipEventRecord(c.stage_ev[size_t(q % slots)], c.stream));
+    };
+    for (int q = 0; q < slots; q++) issue(q);
+    std::mutex mu;  // one thread launches and records at a time
+    std::exception_ptr failed;
+    std::atomic<bool> stop{false};
+    // copier t takes pieces t, t + copiers, ...; a slot belongs to one copier
+    // (slots is a multiple of copiers, or every piece has its own slot)
+    auto copier = [&](int t) {
+        try {
+            MDD_HIP(hipSetDevice(c.device));
+            for (int q = t; q < np && !stop.load(); q += copiers) {
+                MDD_HIP(hipEventSynchronize(c.stage_ev[size_t(q % slots)]));
+                place(pieces[size_t(q)], s + size_t(q % slots) * kSlot);
+                if (q + slots < np) {
+                    std::lock_guard<std::mutex> lk(mu);
+                    issue(q + slots);
+                }
+            }
+        } catch (...) {
+            std::lock_guard<std::mutex> lk(mu);
+            if (!failed) failed = std::current_exception();
+            stop.store(true);
+        }
+    };
+    std::vector<std::thread> threads;
+    try {
+        for (int t = 1; t < copiers; t++) threads.emplace_back(copier, t);
+    } catch (...) {  // no more threads to be had
+        std::lock_guard<std::mutex> lk(mu);
+        failed = std::current_exception();
+        stop.store(true);
+    }
+    if (!stop.load()) copier(0);
+    for (auto& th : threads) th.join();
+    if (failed) {
+        (void)hipStreamSynchronize(c.stream);
+        std::rethrow_exception(failed);
+    }
+}
+
+}  // namespace mdd
