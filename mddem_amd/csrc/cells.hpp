@@ -33,6 +33,14 @@ __device__ inline double readlane_f64(double v, int l) {
     return __longlong_as_double(static_cast<long long>((uint64_t(hi) << 32) | lo));
 }
 
+// orders the wavefront's LDS accesses on either side (lanes read what other
+// lanes of the same wavefront wrote)
+__device__ inline void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Runs of equal keys inside a wavefront: the lane of the run head (h) and
 // of the run tail (t). Invalid lanes form runs of their own.
 __device__ inline void wave_runs(uint32_t key, bool valid, int& h, int& t) {

@@ -366,6 +366,8 @@ struct Ctx {
     bool setup_done = false;
     double max_cutoff = 0, ghost_cutoff = 0, bin_size[3] = {1, 1, 1};
     GridP grid{};
+    int bin_margin = 0;        // bins along x on either side of the box
+    double bins_in_box = 1.0;  // bins of the box itself
     bool uniform = true;
     double cutoff_sq = 0, sf2 = 1, min_skin = 0;
     Shift27 shifts{};

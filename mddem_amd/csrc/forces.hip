@@ -1420,14 +1420,6 @@ struct WaveQueue {
     uint32_t lk[2 * kWaveQ];  // lane | row position << 8 | spring held << 16
 };
 
-// orders the wavefront's LDS accesses on either side (lanes read what other
-// lanes of the same wavefront wrote)
-__device__ inline void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // contact arithmetic of the queued pairs 0..nq-1 (nq <= 64), then each lane
 // adds those it queued (bits of own) to its sums
 template <typename R>

@@ -10,14 +10,14 @@
 // same FP64 fma distance test) comes out bit for bit. Instead of storing
 // only the half list, every particle gets a full row: the pairs it owns
 // plus the pairs other particles own with it, each entry flagged, so the
-// force kernels gather without atomics. Rows are built one wavefront per bin
-// cell (k_build_cells): a candidate after the particle in bin order (a
+// force kernels gather without atomics. Rows are built by wavefronts that take
+// a bin cell each (k_build_rows): a candidate after the particle in bin order (a
 // forward cell, or later in the same cell) is a pair the particle owns; a
 // particle before it owns the pair instead, and for two particles the
 // distance test is symmetric bit for bit. Pairs owned through a particle's
 // periodic images are collected by the images themselves and appended to
 // the particle's row. Passing candidates are compacted with a wavefront
-// ballot, in a fixed order, so rows are deterministic.
+// ballot, in bin order, so rows are deterministic.
 //
 // A batched ensemble shares one cell space: system s owns cells
 // [cell_off, cell_off + ncells) and its own stencil runs and cutoffs.
@@ -354,6 +354,10 @@ struct CellArgs {
     const SysP* __restrict__ sysp;
     const int64_t* __restrict__ sys_cell_off;
     int nsys;
+    // cells [inner_first, inner_first + inner_cells) hold the particles (and
+    // the images beside them); inner_blocks of the launch work through them
+    int64_t inner_first, inner_cells;
+    uint32_t inner_blocks;
     // tile rows (LJ): 16-bit candidate indices, laid out per cell by tile_addr
     uint16_t* __restrict__ crow;
     const uint32_t* __restrict__ lstart;  // first particle of each cell
@@ -387,24 +391,21 @@ struct Window {
     uint64_t okp[kNch];
 };
 
-// Pair tests of one particle of the cell (flat index fs relative to the
-// window) against the window. Candidates before it in bin order own the
-// pair with it (entry flagged), candidates after it are pairs it owns.
-//
-// TILE: the row is written as 16-bit indices into the cell's candidate list
-// (flat index win + 64 c + lane) at tile_addr(s0, cap, M, Gt, m, k), for the
-// tile force kernel; tg = (s0, M, Gt, m, 65536 / Gt rounded up).
+// The tile force kernel's rows are 16-bit indices into the cell's candidate
+// list (flat index win + 64 c + lane) at tile_addr(s0, cap, M, G, m, k).
 struct TileMember {
-    uint32_t s0, M, G, m, ginv;
+    uint32_t s0, M, G, m, ginv;  // ginv: 65536 / G rounded up
 };
 
-template <bool UNIFORM, bool TILE>
+// Pair tests of one particle of the cell (flat index fs relative to the
+// window) against the window. Candidates before it in bin order own the
+// pair with it, candidates after it are pairs it owns.
+template <bool UNIFORM>
 __device__ inline void test_particle(const CellArgs& a, const CellCut& cc,
                                      const Window<UNIFORM>& W, int nch, int fs, const double4& xi,
-                                     uint32_t q, uint32_t& cnt, uint32_t& nrev, uint32_t win,
+                                     uint32_t& cnt, uint32_t& nrev, uint32_t win,
                                      const TileMember& tm) {
     const int lane = int(threadIdx.x & 63);
-    const uint32_t G = 1u << a.lg;
 #pragma unroll
     for (int c = 0; c < kNch; c++) {
         if (c < nch) {
@@ -417,19 +418,10 @@ __device__ inline void test_particle(const CellArgs& a, const CellCut& cc,
                 const uint64_t before = __ballot(f < fs);
                 const uint32_t k = cnt + lanes_before(pass);
                 if (__builtin_amdgcn_inverse_ballot_w64(pass) && k < uint32_t(a.maxnb)) {
-                    if (TILE) {
-                        const uint32_t kq = (k * tm.ginv) >> 16;  // k / G (k < 2^15)
-                        const uint32_t at = tm.s0 * uint32_t(a.tile_cap) + kq * (tm.M * tm.G) +
-                                            tm.m * tm.G + (k - kq * tm.G);
-                        a.crow[at] = uint16_t(win + uint32_t(f));
-                    } else {
-                        // row_addr with 24-bit multiplies (npad < 2^24 is checked by the host)
-                        const uint32_t at = ((__umul24(k >> a.lg, uint32_t(a.npad)) + q) << a.lg) +
-                                            (k & (G - 1u));
-                        a.nbr[at] = __builtin_amdgcn_inverse_ballot_w64(before)
-                                        ? (W.e[c] | kRevBit)
-                                        : W.e[c];
-                    }
+                    const uint32_t kq = (k * tm.ginv) >> 16;  // k / G (k < 2^15)
+                    const uint32_t at = tm.s0 * uint32_t(a.tile_cap) + kq * (tm.M * tm.G) +
+                                        tm.m * tm.G + (k - kq * tm.G);
+                    a.crow[at] = uint16_t(win + uint32_t(f));
                 }
                 cnt += uint32_t(__popcll(pass));
                 nrev += uint32_t(__popcll(pass & before));
@@ -468,51 +460,25 @@ __device__ inline void test_image(const CellArgs& a, const CellCut& cc,
     }
 }
 
-// Neighbor rows, one wavefront per bin cell. The cell's stencil cells form
-// a few runs of consecutive cells, i.e. contiguous bin ranges; concatenated
-// they are the cell's candidate list, whose order is bin order. Candidates
-// are loaded 64 per chunk into registers once, and every member of the cell
-// (particles, then periodic images) is tested against them with uniform
-// control flow; passing lanes are compacted with a ballot, so each row lists
-// its entries in bin order.
-//
-// In a batched ensemble (BATCH) the cell space is shared: the wave finds its
-// cell's system and uses that system's cell range, stencil runs and cutoff.
-template <bool UNIFORM, bool BATCH, bool TILE>
-__global__ void __launch_bounds__(256) k_build_cells(CellArgs a) {
+// Rows for the tile force kernel, one wavefront per bin cell: candidates 64 per
+// chunk in registers, every member of the cell (particles, then periodic
+// images) tested against them with uniform control flow, passing lanes
+// compacted with a ballot.
+template <bool UNIFORM>
+__global__ void __launch_bounds__(256) k_build_tiles(CellArgs a) {
     const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
     const int lane = int(threadIdx.x & 63);
     const int64_t C = int64_t(xcd_block(blockIdx.x, gridDim.x)) * kCellWaves + w;
     if (C >= a.ncells) return;
     const uint32_t i0 = a.bin_start[C], i1 = a.bin_start[C + 1];
     if (i0 == i1) return;
-    int64_t cmin = 0, cmax = a.ncells - 1;
-    int run_off = 0, nruns = a.nruns, run0 = a.run0;
-    CellCut cc{a.cutoff_sq, a.sf2, UNIFORM ? 1 : 0};
-    if (BATCH) {
-        // the system whose cell range holds C
-        int lo = 0, hi = a.nsys - 1;
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (a.sys_cell_off[mid] <= C)
-                lo = mid;
-            else
-                hi = mid - 1;
-        }
-        const SysP& S = a.sysp[lo];
-        cmin = S.cell_off;
-        cmax = S.cell_off + S.grid.ncells - 1;
-        run_off = S.run_off;
-        nruns = S.nruns;
-        run0 = S.run0;
-        cc.cut2 = S.cutoff_sq;
-        cc.sf2 = S.sf2;
-        cc.uni = S.uniform;
-    }
+    const int64_t cmin = 0, cmax = a.ncells - 1;
+    const int nruns = a.nruns, run0 = a.run0;
+    const CellCut cc{a.cutoff_sq, a.sf2, UNIFORM ? 1 : 0};
     // stencil runs in lanes: bin range [rb, rb + rcnt), flat offset excl
     uint32_t rcnt = 0, rb = 0;
     if (lane < nruns) {
-        int64_t lo = C + a.run_first[run_off + lane], hi = C + a.run_last[run_off + lane];
+        int64_t lo = C + a.run_first[lane], hi = C + a.run_last[lane];
         if (lo < cmin) lo = cmin;
         if (hi > cmax) hi = cmax;
         if (lo <= hi) {
@@ -533,14 +499,12 @@ __global__ void __launch_bounds__(256) k_build_cells(CellArgs a) {
     // flat indices of this cell's first slot and of the slot after it
     const int f_i0 = int(i0 - base0), f_i1 = int(i1 - base0);
     const uint32_t ni = i1 - i0;
-    TileMember tm{0u, 0u, 1u, 0u, 65536u};
-    if (TILE) {
-        tm.s0 = a.lstart[C];
-        tm.M = a.lstart[C + 1] - tm.s0;
-        tm.G = uint32_t(tile_lanes(tm.M));
-        tm.ginv = (65536u + tm.G - 1u) / tm.G;
-        if (total > 65535u) atomicOr(&a.st->overflow, 8u);  // tile index range
-    }
+    TileMember tm;
+    tm.s0 = a.lstart[C];
+    tm.M = a.lstart[C + 1] - tm.s0;
+    tm.G = uint32_t(tile_lanes(tm.M));
+    tm.ginv = (65536u + tm.G - 1u) / tm.G;
+    if (total > 65535u) atomicOr(&a.st->overflow, 8u);  // tile index range
     for (uint32_t ib = 0; ib < ni; ib += 64) {
         const uint32_t nib = ni - ib < 64u ? ni - ib : 64u;
         uint32_t cntv = 0, revv = 0;  // lane l: member ib + l
@@ -599,7 +563,6 @@ __global__ void __launch_bounds__(256) k_build_cells(CellArgs a) {
             const int nch = left < uint32_t(kNch) ? int(left) : kNch;
             const int shift = int(win);
             for (uint32_t ii = 0; ii < nloc; ii++) {
-                const uint32_t ei = uint32_t(__builtin_amdgcn_readlane(int(me), int(ii)));
                 double4 xi;
                 xi.x = readlane_f64(mx.x, int(ii));
                 xi.y = readlane_f64(mx.y, int(ii));
@@ -608,9 +571,8 @@ __global__ void __launch_bounds__(256) k_build_cells(CellArgs a) {
                 uint32_t cnt = __builtin_amdgcn_readlane(cntv, int(ii));
                 uint32_t nrev = __builtin_amdgcn_readlane(revv, int(ii));
                 const int fs = f_i0 + int(ib + ii) - shift;
-                if (TILE) tm.m = ib + ii;
-                test_particle<UNIFORM, TILE>(a, cc, W, nch, fs, xi, entry_idx(ei), cnt, nrev, win,
-                                             tm);
+                tm.m = ib + ii;
+                test_particle<UNIFORM>(a, cc, W, nch, fs, xi, cnt, nrev, win, tm);
                 if (uint32_t(lane) == ii) {
                     cntv = cnt;
                     revv = nrev;
@@ -641,10 +603,405 @@ __global__ void __launch_bounds__(256) k_build_cells(CellArgs a) {
     }
 }
 
+// Neighbor rows: the cell's stencil cells form a few runs of consecutive cells,
+// i.e. contiguous bin ranges; concatenated they are the cell's candidate list,
+// whose order is bin order, and each row lists its entries in that order. A
+// wavefront takes a cell (several share its members in small systems), its
+// candidates 64 to a chunk in registers:
+//
+//  1. every member of the cell (particles, then periodic images) is tested
+//     against every chunk with uniform control flow, and the passing lanes
+//     append their candidate index to the member's list in LDS;
+//  2. the lists become entries on their way out: a lane takes 16 bytes of one
+//     row, consecutive lanes consecutive members, which is how the rows are
+//     laid out, so that the stores are whole lines.
+//
+// 87% of the tests fail: what counts is the instructions per 64 tests. Forming
+// each hit's entry, owner flag and row address where it passes took 20 vector
+// and 15 scalar ones; the index alone takes 11 and 10. A particle passes its
+// own test and finds itself in its list, where the entries before it (pairs
+// the other particle owns) end. 256,000 LJ atoms: 117 us (43.2 M vector and
+// 26.6 M scalar instructions) against 165 us (56.5 M and 32.8 M) for rows
+// written entry by entry as they are found; 4,000 atoms 35 against 58 us, the
+// cells shared by four wavefronts. Issue of the tests bounds it.
+//
+// In a batched ensemble (BATCH) the cell space is shared: the wave finds its
+// cell's system and uses that system's cell range, stencil runs and cutoff.
+constexpr int kStage = 2944;  // list slots in LDS per wavefront
+
+// The lists are appended to unchecked: one that outgrows its slots runs into
+// those of the next member, which are written later, and the last one's into
+// the tail, at most one slot per candidate, where the members' data goes
+// afterwards. NCH: chunks of candidates.
+template <int NCH>
+struct RowStage {
+    uint16_t list[kStage];
+    union {
+        uint16_t tail[NCH * 64];
+        struct {
+            uint4 mem[64];    // row length, own place, slot below which w is added
+            uint32_t id[64];  // particle or image
+        };
+    };
+    uint32_t ent[NCH * 64];  // bin slots, then entries, of the candidates
+};
+// four blocks (16 wavefronts) share a CU's 160 KB
+static_assert(kCellWaves * sizeof(RowStage<10>) * 4 <= 160 * 1024, "four blocks per CU");
+
+// Append f of the lanes in `pass` (wavefront-uniform) to the list whose end is
+// the LDS byte address `at` (uniform), which advances. Written as one block
+// with the lanes set by it: from C++ the running end became a vector register
+// and each append a divergent branch, 24 vector instructions per 64 tests. (The
+// two scalar moves are also the two wait states between the compare that wrote
+// `pass` and the first vector read of it.)
+__device__ __forceinline__ void append(uint64_t pass, uint32_t& at, uint32_t f) {
+    uint64_t all;
+    uint32_t t, n;
+    __asm__ volatile(
+        "s_mov_b64 %1, exec\n\t"
+        "s_mov_b64 exec, %4\n\t"
+        "v_mbcnt_lo_u32_b32 %0, %5, 0\n\t"
+        "v_mbcnt_hi_u32_b32 %0, %6, %0\n\t"
+        "v_lshl_add_u32 %0, %0, 1, %3\n\t"
+        "ds_write_b16 %0, %7\n\t"
+        "s_mov_b64 exec, %1\n\t"
+        "s_bcnt1_i32_b64 %2, %4\n\t"
+        "s_lshl1_add_u32 %3, %2, %3"
+        : "=&v"(t), "=&s"(all), "=&s"(n), "+s"(at)
+        : "s"(pass), "s"(uint32_t(pass)), "s"(uint32_t(pass >> 32)), "v"(f)
+        : "memory", "scc");
+}
+
+// f(0), f(1), ... f(N - 1) with the index a constant
+template <int N, int c = 0, typename F>
+__device__ __forceinline__ void each_chunk(F&& f) {
+    if constexpr (c < N) {
+        f(std::integral_constant<int, c>{});
+        each_chunk<N, c + 1>(f);
+    }
+}
+
+template <bool UNIFORM, bool BATCH, int NCH>
+__global__ void __launch_bounds__(256) k_build_rows(CellArgs a, int wpc_log2) {
+    constexpr uint32_t kWin = NCH * 64;
+    __shared__ RowStage<NCH> stage[kCellWaves];
+    const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+    const int lane = int(threadIdx.x & 63);
+    RowStage<NCH>& L = stage[w];
+    // blocks of the cells that hold particles first, each XCD a contiguous
+    // range of them, then those of the image layers at both ends, much lighter
+    const bool inner = blockIdx.x < a.inner_blocks;
+    const uint32_t blk = inner ? xcd_block(blockIdx.x, a.inner_blocks)
+                               : blockIdx.x - a.inner_blocks;
+    const int64_t wave = int64_t(blk) * kCellWaves + w;
+    int64_t C = wave >> wpc_log2;
+    const uint32_t share = uint32_t(wave & ((1 << wpc_log2) - 1));
+    if (inner) {
+        if (C >= a.inner_cells) return;
+        C += a.inner_first;
+    } else {
+        if (C >= a.inner_first) C += a.inner_cells;
+        if (C >= a.ncells) return;
+    }
+    const uint32_t i0 = a.bin_start[C], i1 = a.bin_start[C + 1];
+    // this wavefront's members of the cell
+    const uint32_t m0 = ((i1 - i0) * share) >> wpc_log2;
+    const uint32_t m1 = ((i1 - i0) * (share + 1u)) >> wpc_log2;
+    if (m0 == m1) return;
+    int64_t cmin = 0, cmax = a.ncells - 1;
+    int run_off = 0, nruns = a.nruns, run0 = a.run0;
+    CellCut cc{a.cutoff_sq, a.sf2, UNIFORM ? 1 : 0};
+    if (BATCH) {
+        // the system whose cell range holds C
+        int lo = 0, hi = a.nsys - 1;
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (a.sys_cell_off[mid] <= C)
+                lo = mid;
+            else
+                hi = mid - 1;
+        }
+        const SysP& S = a.sysp[lo];
+        cmin = S.cell_off;
+        cmax = S.cell_off + S.grid.ncells - 1;
+        run_off = S.run_off;
+        nruns = S.nruns;
+        run0 = S.run0;
+        cc.cut2 = S.cutoff_sq;
+        cc.sf2 = S.sf2;
+        cc.uni = S.uniform;
+    }
+    // stencil runs in lanes: bin range [rb, rb + rcnt), flat offset excl
+    uint32_t rcnt = 0, rb = 0;
+    if (lane < nruns) {
+        int64_t lo = C + a.run_first[run_off + lane], hi = C + a.run_last[run_off + lane];
+        if (lo < cmin) lo = cmin;
+        if (hi > cmax) hi = cmax;
+        if (lo <= hi) {
+            rb = a.bin_start[lo];
+            rcnt = a.bin_start[hi + 1] - rb;
+        }
+    }
+    uint32_t incl = rcnt;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t t = __shfl_up(incl, d, 64);
+        if (lane >= d) incl += t;
+    }
+    const uint32_t excl = incl - rcnt;
+    uint32_t total = __builtin_amdgcn_readlane(incl, nruns - 1);
+    // flat indices of this cell's first slot and of the slot after it
+    const int f_i0 = int(i0 - uint32_t(__builtin_amdgcn_readlane(rb - excl, run0)));
+    const int f_i1 = f_i0 + int(i1 - i0);
+    // A cell outside the box holds images only, which pair with the particles
+    // up to the end of their cell: the list ends there, and half of these
+    // cells (those below the box in bin order) have no such particle at all.
+    if (a.lstart[C] == a.lstart[C + 1]) {
+        total = uint32_t(f_i1);
+        uint32_t np = 0u;
+        if (lane <= run0) {
+            int64_t lo = C + a.run_first[run_off + lane], hi = C + a.run_last[run_off + lane];
+            if (lo < cmin) lo = cmin;
+            if (hi > C) hi = C;
+            if (lo <= hi) np = a.lstart[hi + 1] - a.lstart[lo];
+        }
+        if (__ballot(np != 0u) == 0ull) {
+            for (uint32_t m = m0 + uint32_t(lane); m < m1; m += 64u)
+                a.gcnt[a.bin_gidx[i0 + m]] = 0u;
+            return;
+        }
+    }
+    const uint32_t maxnb = uint32_t(a.maxnb);
+    // a list holds a full row and the particle itself; an odd number of words
+    const uint32_t pitch = (maxnb + 2u) | 2u;
+    // one window, at least one list in LDS and members of one kind (a particle
+    // and an image share a cell only where rounding puts an image inside the
+    // box), else each entry goes straight to memory as it is found
+    const uint32_t np_cell = a.lstart[C + 1] - a.lstart[C];
+    const bool images = np_cell == 0u;
+    const bool staged = total <= kWin && pitch <= uint32_t(kStage) &&
+                        (images || np_cell == i1 - i0);
+    uint32_t cap = staged ? uint32_t(kStage) / pitch : 64u;
+    if (cap > 64u) cap = 64u;
+    const uint32_t M = m1 - m0;
+    const uint32_t nbat = (M + cap - 1u) / cap;
+    const uint32_t per = (M + nbat - 1u) / nbat;  // even batches
+    double X[NCH], Y[NCH], Z[NCH], R[UNIFORM ? 1 : NCH];
+    if (UNIFORM) R[0] = 0.0;
+    uint32_t some = 0u;  // bit c: chunk c has candidates
+    // The candidates: for particles every particle, and every periodic image
+    // that is not in a backward cell (those pairs belong to the image's
+    // particle, found through its own images); for images the particles up to
+    // the end of their cell. The others are put out of reach.
+    if (staged) {
+        for (int r = 0; r < nruns; r++) {
+            const uint32_t n_r = __builtin_amdgcn_readlane(rcnt, r);
+            const uint32_t x_r = __builtin_amdgcn_readlane(excl, r);
+            const uint32_t b_r = __builtin_amdgcn_readlane(rb, r);
+            for (uint32_t t = uint32_t(lane); t < n_r && x_r + t < kWin; t += 64u)
+                L.ent[x_r + t] = b_r + t;
+        }
+        wave_lds_sync();
+        // every chunk's loads are issued before any is used (lanes past the
+        // list read slot 0 and are masked off), so the window costs one
+        // memory latency rather than one per chunk
+        uint32_t ev[NCH];
+#pragma unroll
+        for (int c = 0; c < NCH; c++) {
+            const uint32_t f = uint32_t(c * 64 + lane);
+            const uint32_t src = f < total ? L.ent[f] : 0u;
+            const double4 q = a.bin_pos[src];
+            X[c] = q.x;
+            Y[c] = q.y;
+            Z[c] = q.z;
+            if (!UNIFORM) R[c] = q.w;
+            ev[c] = a.bin_entry[src];
+        }
+        each_chunk<NCH>([&](auto ic) {
+            constexpr int c = decltype(ic)::value;
+            const uint32_t f = uint32_t(c * 64 + lane);
+            const bool particle = entry_code(ev[c]) == kCodeNone;
+            const bool ok = f < total && (images ? particle && int(f) < f_i1
+                                                 : particle || int(f) >= f_i0);
+            if (!ok) X[c] = 1e150;
+            some |= __ballot(ok) != 0ull ? 1u << c : 0u;
+            L.ent[c * 64 + lane] = ev[c];
+        });
+    }
+    for (uint32_t b0 = m0; b0 < m1; b0 += per) {
+        const uint32_t nb = m1 - b0 < per ? m1 - b0 : per;
+        // the batch's members, lane l holding member b0 + l
+        double4 mx = make_double4(0.0, 0.0, 0.0, 0.0);
+        uint32_t me = 0u, mg = 0u;
+        if (uint32_t(lane) < nb) {
+            const uint32_t slot = i0 + b0 + uint32_t(lane);
+            mx = a.bin_pos[slot];
+            me = a.bin_entry[slot];
+            if (entry_code(me) != kCodeNone) mg = a.bin_gidx[slot];
+        }
+        const bool mimg = entry_code(me) != kCodeNone;
+        // members 0 .. nloc - 1 are particles (they precede the images)
+        const uint32_t nloc = uint32_t(__popcll(__ballot(uint32_t(lane) < nb && !mimg)));
+        // what is added to an entry below flat index mfs: the owner flag
+        // (particles: the partners before their own slot own those pairs), and
+        // for an image its code in place of the partner's
+        const uint32_t mset =
+            mimg ? kRevBit + (uint32_t(entry_code(me) - kCodeNone) << kIdxBits) : kRevBit;
+        const uint32_t mfs = mimg ? 0xFFFFFFFFu : uint32_t(f_i0) + b0 + uint32_t(lane);
+        uint32_t mcnt = 0u, mrev = 0u;
+        if (staged) {
+            wave_lds_sync();
+            const uint32_t list0 = uint32_t(reinterpret_cast<uintptr_t>(
+                (__attribute__((address_space(3))) void*)(L.list)));
+            for (uint32_t j = 0; j < nb; j++) {
+                const double xi = readlane_f64(mx.x, int(j)), yi = readlane_f64(mx.y, int(j)),
+                             zi = readlane_f64(mx.z, int(j)),
+                             ri = UNIFORM ? 0.0 : readlane_f64(mx.w, int(j));
+                const uint32_t begin = __builtin_amdgcn_readfirstlane(list0 + 2u * j * pitch);
+                uint32_t at = begin, live = some;
+                // (opaque: else the ten branch conditions are kept in scalar
+                // register pairs, which run out)
+                __asm__ volatile("" : "+s"(live));
+                each_chunk<NCH>([&](auto ic) {
+                    constexpr int c = decltype(ic)::value;
+                    if (!((live >> c) & 1u)) return;
+                    const double dx = X[c] - xi, dy = Y[c] - yi, dz = Z[c] - zi;
+                    const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
+                    append(__ballot(within<UNIFORM>(cc, r2, ri, R[UNIFORM ? 0 : c])), at,
+                           uint32_t(c * 64 + lane));
+                });
+                if (uint32_t(lane) == j) mcnt = (at - begin) >> 1;
+            }
+            wave_lds_sync();
+            // the particle's own place in its list (a list is ascending)
+            const uint32_t have = mcnt < pitch ? mcnt : pitch;
+            uint32_t self = 0xFFFFFFFFu;
+            if (uint32_t(lane) < nloc) {
+                uint32_t lo = 0u, hi = have;
+                while (lo < hi) {
+                    const uint32_t mid = (lo + hi) >> 1;
+                    if (uint32_t(L.list[uint32_t(lane) * pitch + mid]) < mfs)
+                        lo = mid + 1u;
+                    else
+                        hi = mid;
+                }
+                mrev = lo;
+                // (counted whether or not it fitted: a count above maxnb asks
+                // for rows of that length)
+                if (within<UNIFORM>(cc, 0.0, mx.w, mx.w)) {
+                    self = lo;
+                    mcnt--;
+                }
+            }
+            // the rows, V words (16 bytes, or the layout's contiguous entries)
+            // at a time: unit u of member m
+            const uint32_t out = mcnt < maxnb ? mcnt : maxnb;
+            uint32_t most = out;
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) {
+                const uint32_t t = __shfl_xor(most, o, 64);
+                most = t > most ? t : most;
+            }
+            const uint32_t vlg = a.lg < 2 ? uint32_t(a.lg) : 2u;
+            const uint32_t units = ((most + (1u << vlg) - 1u) >> vlg) * nb;
+            if (uint32_t(lane) < nb) {
+                L.mem[lane] = make_uint4(out, self, mfs, mset);
+                L.id[lane] = mimg ? mg : entry_idx(me);
+            }
+            wave_lds_sync();
+            const float inv = 1.0f / float(nb);
+            for (uint32_t t = uint32_t(lane); t < units; t += 64u) {
+                // t / nb for t < 2^16: the quotient of the middle of the step
+                const uint32_t u = uint32_t((float(t) + 0.5f) * inv), m = t - u * nb;
+                const uint4 q = L.mem[m];
+                const uint32_t id = L.id[m];
+                const uint32_t k = u << vlg;
+                if (k >= q.x) continue;
+                const uint16_t* list = L.list + m * pitch;
+                // the entry of list position kk (image members' partners are
+                // particles, whose entries have the code of no image: the
+                // difference turns it into the image's)
+                auto entry = [&](uint32_t kk) {
+                    const uint32_t f = list[kk >= q.y ? kk + 1u : kk];
+                    return L.ent[f] + (f < q.z ? q.w : 0u);
+                };
+                // (32-bit row indices, 24-bit factors: checked by the host)
+                const uint32_t at =
+                    ((__umul24(k >> a.lg, uint32_t(a.npad)) + id) << a.lg) + (k & ((1u << a.lg) - 1u));
+                uint32_t* to = m < nloc ? a.nbr + at : a.gnbr + size_t(id) * maxnb + k;
+                const uint32_t last = q.x - 1u;  // words past the row repeat its last entry
+                if (vlg == 2u) {
+                    const uint32_t k1 = k + 1u < last ? k + 1u : last;
+                    const uint32_t k2 = k + 2u < last ? k + 2u : last;
+                    const uint32_t k3 = k + 3u < last ? k + 3u : last;
+                    *reinterpret_cast<uint4*>(to) =
+                        make_uint4(entry(k), entry(k1), entry(k2), entry(k3));
+                } else if (vlg == 1u) {
+                    *reinterpret_cast<uint2*>(to) =
+                        make_uint2(entry(k), entry(k < last ? k + 1u : k));
+                } else {
+                    *to = entry(k);
+                }
+            }
+        } else {
+            // candidates 64 at a time, straight from memory
+            for (uint32_t f0 = 0; f0 < total; f0 += 64u) {
+                const uint32_t f = f0 + uint32_t(lane);
+                uint32_t src = 0u;
+                for (int r = 0; r < nruns; r++) {
+                    const uint32_t x_r = __builtin_amdgcn_readlane(excl, r);
+                    const uint32_t b_r = __builtin_amdgcn_readlane(rb, r);
+                    if (f < total && f >= x_r) src = b_r + (f - x_r);
+                }
+                const double4 q = a.bin_pos[src];
+                const uint32_t e = a.bin_entry[src];
+                const bool particle = f < total && entry_code(e) == kCodeNone;
+                const bool ok_p = particle || (f < total && int(f) >= f_i0);
+                const bool ok_i = particle && int(f) < f_i1;
+                for (uint32_t j = 0; j < nb; j++) {
+                    const double dx = q.x - readlane_f64(mx.x, int(j)),
+                                 dy = q.y - readlane_f64(mx.y, int(j)),
+                                 dz = q.z - readlane_f64(mx.z, int(j));
+                    const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
+                    const uint32_t fs = __builtin_amdgcn_readlane(mfs, int(j));
+                    const bool in = within<UNIFORM>(cc, r2, readlane_f64(mx.w, int(j)), q.w) &&
+                                    f != fs && (j < nloc ? ok_p : ok_i);
+                    const uint64_t pass = __ballot(in);
+                    if (pass == 0ull) continue;
+                    const uint32_t id =
+                        __builtin_amdgcn_readlane(mimg ? mg : entry_idx(me), int(j));
+                    const uint32_t set = __builtin_amdgcn_readlane(mset, int(j));
+                    const uint32_t k =
+                        __builtin_amdgcn_readlane(mcnt, int(j)) + lanes_before(pass);
+                    if (in && k < maxnb) {
+                        const uint32_t x = e + (f < fs ? set : 0u);
+                        if (j >= nloc)
+                            a.gnbr[size_t(id) * maxnb + k] = x;
+                        else
+                            a.nbr[row_addr(int64_t(id), int(k), a.npad, a.lg)] = x;
+                    }
+                    if (uint32_t(lane) == j) {
+                        mcnt += uint32_t(__popcll(pass));
+                        if (fs != 0xFFFFFFFFu) mrev += uint32_t(__popcll(pass & lanes_below(int(fs) - int(f0))));
+                    }
+                }
+            }
+        }
+        if (uint32_t(lane) < nb) {
+            if (mimg) {
+                a.gcnt[mg] = mcnt;
+            } else {
+                a.nnb[entry_idx(me)] = mcnt;
+                a.nhalf[entry_idx(me)] = mcnt - mrev;
+            }
+        }
+    }
+}
+
 // The same rows for sparse grids (most cells empty or nearly so, where a
 // wavefront per cell idles): one lane per member slot, walking its cell's
 // stencil runs in bin order. Candidate order, the ownership flags and the
-// counts are those of k_build_cells, so the rows are identical.
+// counts are those of k_build_rows, so the rows are identical.
 template <bool UNIFORM>
 __global__ void __launch_bounds__(256) k_build_sparse(CellArgs a,
                                                       const uint32_t* __restrict__ bin_cell,
@@ -1318,6 +1675,15 @@ void rebuild_prepare(Ctx& c) {
     c.lg_old = c.list_lg;
 }
 
+// log2 of the wavefronts that share a cell's members in k_build_rows. Each of
+// them reads the cell's candidates, so sharing pays while the cells alone leave
+// the chip's 4096 wavefront places (256 CUs x 16) idle. Whole rebuilds of LJ
+// fluids with 1, 2 and 4 wavefronts per cell, in us: 4,000 atoms (216 cells)
+// 121, 98, 91; 11,000 104, 94, 92; 20,000 (850 cells) 114, 104, 105; 49,000
+// (2,100) 147, 139, 151; 144,000 (6,200) 203, 198, 205; 256,000 (11,000) 263,
+// 261, 284; 500,000 (21,600) 376, 400, 473.
+int build_waves_log2(double cells) { return cells < 896.0 ? 2 : (cells < 10240.0 ? 1 : 0); }
+
 // one build of images, bins and rows with the current capacities; the
 // status says afterwards whether everything fitted
 void rebuild_attempt(Ctx& c) {
@@ -1425,16 +1791,35 @@ void rebuild_attempt(Ctx& c) {
         launch(c, k_build_sparse<false>, blocks_for(nall_max, 256), 256, ca,
                static_cast<const uint32_t*>(c.bin_cell.p), static_cast<const uint32_t*>(ng_live),
                n);
-    else if (c.nsys > 0)
-        launch(c, k_build_cells<false, true, false>, cblocks, 256, ca);
     else if (tile && c.uniform)
-        launch(c, k_build_cells<true, false, true>, cblocks, 256, ca);
+        launch(c, k_build_tiles<true>, cblocks, 256, ca);
     else if (tile)
-        launch(c, k_build_cells<false, false, true>, cblocks, 256, ca);
-    else if (c.uniform)
-        launch(c, k_build_cells<true, false, false>, cblocks, 256, ca);
-    else
-        launch(c, k_build_cells<false, false, false>, cblocks, 256, ca);
+        launch(c, k_build_tiles<false>, cblocks, 256, ca);
+    else {
+        const int wl = build_waves_log2(c.nsys > 0 ? double(ncells) : c.bins_in_box);
+        // single systems: the x layers inside the image margin
+        const int64_t layer = int64_t(c.grid.n[1]) * c.grid.n[2];
+        const int64_t margin = c.nsys > 0 ? 0 : c.bin_margin;
+        ca.inner_first = margin * layer;
+        ca.inner_cells = ncells - 2 * ca.inner_first;
+        ca.inner_blocks = uint32_t(blocks_for(ca.inner_cells << wl, kCellWaves));
+        const int rblocks = int(ca.inner_blocks) +
+                            int((((2 * ca.inner_first) << wl) + kCellWaves - 1) / kCellWaves);
+        // candidates of a cell at the mean density, with a tenth to spare: 640
+        // fit 10 chunks at 4 wavefronts per SIMD (LJ fluids: 490 to 600); the
+        // wider bins of a box of few cells need 16, at 3 wavefronts (4,000
+        // atoms: 5 bins a side, 860 candidates; from memory instead of
+        // registers such a build takes 58 us instead of 35)
+        const double cand = double(n) / c.bins_in_box * double(c.full.size());
+        if (c.nsys > 0)
+            launch(c, k_build_rows<false, true, 10>, rblocks, 256, ca, wl);
+        else if (c.uniform && cand * 1.1 <= 640.0)
+            launch(c, k_build_rows<true, false, 10>, rblocks, 256, ca, wl);
+        else if (c.uniform)
+            launch(c, k_build_rows<true, false, 16>, rblocks, 256, ca, wl);
+        else
+            launch(c, k_build_rows<false, false, 10>, rblocks, 256, ca, wl);
+    }
     const int tblocks = blocks_for(n, 256);
     c.row_blk.resize(size_t(2) * tblocks);
     launch(c, k_row_totals, tblocks, 256, n, c.goff.p, ng_live, c.gcnt_img.p, c.nmain.p,
@@ -1771,6 +2156,8 @@ struct Geometry {
     int run0 = -1, nfwd = 0;
     bool uniform = true;
     double cutoff_sq = 0, sf2 = 1, min_skin = 0;
+    int margin = 0;  // bins along x on either side of the box
+    double in_box = 1.0;  // bins of the box itself
 };
 
 Geometry make_geometry(const BoxP& box, double mn, double mx, double skin_fraction,
@@ -1800,6 +2187,8 @@ Geometry make_geometry(const BoxP& box, double mn, double mx, double skin_fracti
         g.grid.origin[d] = box.lo[d] - g.bin_size[d] * double(sl[d]);
         g.grid.inv_bs[d] = 1.0 / g.bin_size[d];
     }
+    g.margin = sl[0];
+    g.in_box = double(nint[0]) * nint[1] * nint[2];
     g.grid.ncells = int64_t(g.grid.n[0]) * g.grid.n[1] * g.grid.n[2];
     if (g.grid.ncells > (int64_t(1) << 31))
         throw ApiError(-5, "bin grid too large; raise bin_size");
@@ -1917,6 +2306,8 @@ void neighbor_setup(Ctx& c) {
     c.max_cutoff = g.max_cutoff;
     c.ghost_cutoff = g.ghost_cutoff;
     for (int d = 0; d < 3; d++) c.bin_size[d] = g.bin_size[d];
+    c.bin_margin = g.margin;
+    c.bins_in_box = g.in_box;
     c.full = g.full;
     c.nruns = int(g.run_first.size());
     c.run0 = g.run0;
