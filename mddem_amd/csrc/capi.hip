@@ -41,7 +41,7 @@ __global__ void k_status_init(mdd::Status* st) {
     st->overflow = 0u;
     st->third = 0;
     st->max_row = 0;
-    st->max_half = 0;
+    st->rebuild_step = INT_MAX;
     st->ghost_total = 0u;
     st->overlap_count[0] = st->overlap_count[1] = 0;
     st->nh_kind[0] = st->nh_kind[1] = 1;

@@ -233,8 +233,8 @@ struct Status {
                              // bit 3: candidate list beyond 16-bit tile indices
                              // bit 4: more old contacts than history records
     int third;               // rebuild: the state is in the third buffers
-    int max_row;             // longest full-list row at the last build
-    int max_half;            // longest half-list row at the last build
+    int max_row;             // longest full-list row of a build that did not fit
+    int rebuild_step;        // the step of the rebuild under way (INT_MAX: none)
     unsigned ghost_total;    // periodic images at the last build
     int overlap_count[2];    // large-overlap pairs, by step parity
     int nh_kind[2];          // per step parity: 1 = nh_p is p_xi after a post
@@ -431,11 +431,12 @@ struct Ctx {
     DBuf<float> f32b, t32b;
 
     // ---- rebuild scratch
-    DBuf<uint32_t> key, key2, order, slot_of, cnt, start, scan_tmp, gcnt, goff;
+    DBuf<uint32_t> key, key2, order, cnt, start, scan_tmp, gcnt, goff;
+    DBuf<uint32_t> gtot;  // images of every kGhostTile particles
     DBuf<uint32_t> ghost_root;
     DBuf<uint8_t> ghost_code;
     DBuf<double4> ghost_pos;
-    DBuf<uint32_t> bin_start, bin_entry, gstart, placed, ghost_key, ghost_order;
+    DBuf<uint32_t> bin_start, bin_entry, gstart, placed, ghost_key;
     DBuf<double4> bin_pos;
     std::vector<int> full;   // all offsets whose cells can hold a pair, ascending
     DBuf<int> run_first, run_last;  // the full stencil as runs of consecutive offsets
@@ -494,7 +495,6 @@ struct Ctx {
     DBuf<uint16_t> crow;
     DBuf<uint32_t> xnbr, nx;
     DBuf<double> ke_total;          // NH kinetic energy sum for the next pre kernel
-    DBuf<uint32_t> row_blk;         // per-block row maxima of the last build
     DBuf<double> vir;               // energy passes: per-particle virial, 6 x npad
     // DEM contact virial: computed in the force pass of every step whose
     // number is a multiple of virial_every (0: never); vir then holds the
@@ -561,8 +561,7 @@ struct Ctx {
 
     // ---- rebuild launch sequences captured as graphs
     LaunchLog rec;
-    int row_nblk = 0;  // per-block row-maxima slots of the last build
-    // device time of whole rebuilds (first launch to the gate) and of the
+    // device time of whole rebuilds (first launch to last) and of the
     // idle gap before them (end of the step chunk that asked for the rebuild
     // to its first launch), when profiling: events 3k, 3k+1, 3k+2
     std::vector<hipEvent_t> rb_ev;
@@ -588,11 +587,10 @@ struct Ctx {
 
 // ---- launchers implemented in the .hip files
 // scan_sort.hip
-void exclusive_scan(Ctx& c, const uint32_t* in, uint32_t* out, int64_t n);
-void counting_sort(Ctx& c, const uint32_t* key, int64_t n, const uint32_t* n_dev, int64_t ncells,
-                   uint32_t* cnt, uint32_t* start, uint32_t* placed, uint32_t* order,
-                   uint32_t* slot_of, bool cnt_zero = false, const uint32_t* add = nullptr,
-                   uint32_t* out2 = nullptr, bool counted = false);
+void exclusive_scan(Ctx& c, const uint32_t* in, uint32_t* out, int64_t n,
+                    const uint32_t* add = nullptr, uint32_t* out2 = nullptr);
+void place_by_key(Ctx& c, const uint32_t* key, int64_t n, const uint32_t* n_dev,
+                  const uint32_t* start, uint32_t* cnt, uint32_t* placed);
 void fill_u32(Ctx& c, uint32_t* p, uint32_t v, int64_t n);
 void fill_f64(Ctx& c, double* p, double v, int64_t n);
 void fill_f32(Ctx& c, float* p, float v, int64_t n);

@@ -41,23 +41,38 @@ __device__ inline uint32_t cell_of(const GridP& g, double x, double y, double z)
     return uint32_t(cx * g.n[1] * g.n[2] + cy * g.n[2] + cz);
 }
 
-// Start of a rebuild: the step sequence resumes (abort cleared), the build
-// status is reset and the sort's per-cell counts are zeroed. third: which
-// buffers hold the state to sort (a word that the sort's kernels read, so that
-// their arguments, and with them a captured launch sequence, do not depend on it).
+// Start of a build: the step sequence resumes (abort cleared), the build's
+// status is reset and the sort's per-cell counts are zeroed. Launched by
+// itself, ahead of the recorded launches, with what differs from rebuild to
+// rebuild: the step, and which buffers hold the state (third: a word that the
+// sort's kernels read, so that their arguments, and with them a captured launch
+// sequence, do not depend on it). retry: the build of the same sorted state
+// again, larger.
 __global__ void k_rebuild_begin(Status* st, uint32_t* __restrict__ cnt, int64_t ncells,
-                                int third) {
-    for (int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; i < ncells;
-         i += int64_t(gridDim.x) * blockDim.x)
-        cnt[i] = 0u;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        st->third = third;
-        st->abort_step = INT_MAX;
-        st->overflow = 0u;
+                                uint32_t* __restrict__ gtot, int64_t ntiles, int third, int step,
+                                int retry) {
+    const int64_t i0 = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
+    const int64_t stride = int64_t(gridDim.x) * blockDim.x;
+    for (int64_t i = i0; i < ncells; i += stride) cnt[i] = 0u;
+    if (!retry)
+        for (int64_t i = i0; i < ntiles; i += stride) gtot[i] = 0u;
+    if (i0 == 0) {
+        // (a retry keeps the fixed-boundary exit seen by the wrap)
+        const uint32_t keep = retry ? st->overflow & 4u : 0u;
+        if (!retry) st->third = third;
+        st->abort_step = keep ? step : INT_MAX;
+        st->rebuild_step = step;
+        st->overflow = keep;
         st->max_row = 0;
-        st->max_half = 0;
         st->ghost_total = 0u;
     }
+}
+
+// A build that does not fit: the host repeats it with larger capacities when
+// it next reads the status, and the step's later kernels do not run.
+__device__ inline void build_failed(Status* st, uint32_t bit) {
+    atomicOr(&st->overflow, bit);
+    atomicMin(&st->abort_step, st->rebuild_step);
 }
 
 // pbc wrap (wrap_periodic, domain.rs:396-407) + bin key of every particle,
@@ -82,29 +97,29 @@ __global__ void k_wrap_key(int64_t n, double4* pos, double4* pos3, int4* __restr
             coff = S.cell_off;
         }
         double4 p = pos[i];
-        int4 im = image[i];
         double x[3] = {p.x, p.y, p.z};
-        int m[3] = {im.x, im.y, im.z};
+        int m[3] = {0, 0, 0};
 #pragma unroll
         for (int d = 0; d < 3; d++) {
             if (box.periodic[d]) {
                 double high = box.lo[d] + box.L[d];
                 if (x[d] < box.lo[d]) {
                     x[d] += box.L[d];
-                    m[d] += -1;
+                    m[d] = -1;
                 } else if (x[d] >= high) {
                     x[d] -= box.L[d];
-                    m[d] += 1;
+                    m[d] = 1;
                 }
             } else if (x[d] < box.lo[d] || x[d] >= box.hi[d]) {
-                atomicOr(&st->overflow, 4u);  // left a fixed boundary
+                build_failed(st, 4u);  // left a fixed boundary
             }
         }
-        p.x = x[0];
-        p.y = x[1];
-        p.z = x[2];
-        pos[i] = p;
-        image[i] = make_int4(m[0], m[1], m[2], 0);
+        // few particles cross a face between two builds: only those are written
+        if (m[0] | m[1] | m[2]) {
+            pos[i] = make_double4(x[0], x[1], x[2], p.w);
+            const int4 im = image[i];
+            image[i] = make_int4(im.x + m[0], im.y + m[1], im.z + m[2], 0);
+        }
         kc = uint32_t(coff + cell_of(g, x[0], x[1], x[2]));
         key[i] = kc;
     }
@@ -134,49 +149,35 @@ struct PermArgs {
     int4* bxq;  // with xq: the same values as the fixed-point build positions
     double qs[3];
     int dem;
+    // the sort: elements placed in their cells (null: order is given instead)
+    const uint32_t *placed, *start;
+    uint32_t* order_out;
+    // periodic images: count of every particle and of every kGhostTile of them
+    BoxP box;
+    double gc;
+    const SysP* sysp;
+    const uint32_t* psys;
+    uint32_t *gcnt, *gtot;
 };
 
-// apply the sort permutation to every per-particle array (Atom::apply_permutation,
-// atom.rs:383-394) and record the build positions (save_build_positions)
-__global__ void k_permute(PermArgs a) {
-    int64_t k = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-    if (k >= a.n) return;
-    if (a.st->third) {
-        a.pos = a.pos3;
-        a.vel = a.vel3;
-        a.omega = a.omega3;
+// particles per word of gtot
+constexpr int kGhostTileLog2 = 10;
+
+// place of element v, found in slot of its cell's range [b, e) of `placed`:
+// index order inside the cell
+__device__ inline uint32_t cell_rank(const uint32_t* __restrict__ placed, uint32_t b, uint32_t e,
+                                     uint32_t v) {
+    // (eight loads in flight: the lanes of a cell read the same words, so the
+    // latency is what counts)
+    uint32_t r = b;
+    for (uint32_t t = b; t < e; t += 8u) {
+        uint32_t x[8];
+#pragma unroll
+        for (uint32_t j = 0; j < 8u; j++) x[j] = placed[t + j < e ? t + j : b];
+#pragma unroll
+        for (uint32_t j = 0; j < 8u; j++) r += t + j < e && x[j] < v ? 1u : 0u;
     }
-    uint32_t o = a.order[k];
-    double4 p = a.pos[o];
-    a.pos2[k] = p;
-    a.build_pos[k] = p;
-    if (a.xq) {
-        const int4 q = make_int4(quantize_axis(p.x, a.qs[0]), quantize_axis(p.y, a.qs[1]),
-                                 quantize_axis(p.z, a.qs[2]), 0);
-        a.xq[k] = q;
-        a.bxq[k] = q;
-    }
-    a.vel2[k] = a.vel[o];
-    a.tag2[k] = a.tag[o];
-    a.type2[k] = a.type[o];
-    a.key2[k] = a.key[o];
-    a.image2[k] = a.image[o];
-    a.mass2[k] = a.mass[o];
-    a.cutr2[k] = a.cutr[o];
-    if (a.f64) {
-        for (int d = 0; d < 3; d++) a.f64b[d * a.npad + k] = a.f64[d * a.npad + o];
-    }
-    if (a.f32) {
-        for (int d = 0; d < 3; d++) a.f32b[d * a.npad + k] = a.f32[d * a.npad + o];
-    }
-    if (a.dem) {
-        a.omega2[k] = a.omega[o];
-        a.quat2[k] = a.quat[o];
-        if (a.t64)
-            for (int d = 0; d < 3; d++) a.t64b[d * a.npad + k] = a.t64[d * a.npad + o];
-        if (a.t32)
-            for (int d = 0; d < 3; d++) a.t32b[d * a.npad + k] = a.t32[d * a.npad + o];
-    }
+    return r;
 }
 
 // image flags of one particle: which faces it is within the ghost cutoff of
@@ -191,53 +192,148 @@ __device__ inline void image_flags(const BoxP& box, double gc, const double x[3]
     }
 }
 
-// Start of one build attempt (a retry repeats it with larger capacities):
-// status reset and the image sort's per-cell counts zeroed, fused with the
-// image count of every particle.
-__global__ void k_ghost_count(int64_t n, const double4* __restrict__ pos, BoxP box, double gc,
-                              uint32_t* __restrict__ gcnt, const SysP* __restrict__ sysp,
-                              const uint32_t* __restrict__ psys, Status* st,
-                              uint32_t* __restrict__ cnt, int64_t ncells) {
-    for (int64_t c = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; c < ncells;
-         c += int64_t(gridDim.x) * blockDim.x)
-        cnt[c] = 0u;
-    int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-    if (i == 0) {
-        st->abort_step = INT_MAX;
-        st->overflow &= 4u;  // keep the fixed-boundary exit seen by the wrap
-        st->max_row = 0;
-        st->max_half = 0;
-        st->ghost_total = 0u;
+// apply the sort permutation to every per-particle array (Atom::apply_permutation,
+// atom.rs:383-394) and record the build positions (save_build_positions)
+// The last pass of the sort and the first of the images as well: a thread takes
+// a placed element, ranks it inside its cell and moves it there, then counts
+// its periodic images. It moves about 330 B per particle (LJ, mixed), which
+// bounds it: 21 us at 256,000 particles, 8 us at 4,000. As kernels of their own
+// move, rank, image count and its scan took 36 us (5 launches) and 19 us (4).
+template <bool PLACED>
+__global__ void __launch_bounds__(256) k_permute(PermArgs a) {
+    int64_t k = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
+    const bool live = k < a.n;
+    uint32_t images = 0u;
+    if (live) {
+        if (a.st->third) {
+            a.pos = a.pos3;
+            a.vel = a.vel3;
+            a.omega = a.omega3;
+        }
+        uint32_t o;
+        if (PLACED) {
+            o = a.placed[k];
+            const uint32_t cell = a.key[o];
+            k = int64_t(cell_rank(a.placed, a.start[cell], a.start[cell + 1], o));
+            a.order_out[k] = o;
+        } else {
+            o = a.order[k];
+        }
+        double4 p = a.pos[o];
+        a.pos2[k] = p;
+        a.build_pos[k] = p;
+        if (a.xq) {
+            const int4 q = make_int4(quantize_axis(p.x, a.qs[0]), quantize_axis(p.y, a.qs[1]),
+                                     quantize_axis(p.z, a.qs[2]), 0);
+            a.xq[k] = q;
+            a.bxq[k] = q;
+        }
+        a.vel2[k] = a.vel[o];
+        a.tag2[k] = a.tag[o];
+        a.type2[k] = a.type[o];
+        a.key2[k] = a.key[o];
+        a.image2[k] = a.image[o];
+        a.mass2[k] = a.mass[o];
+        a.cutr2[k] = a.cutr[o];
+        if (a.f64) {
+            for (int d = 0; d < 3; d++) a.f64b[d * a.npad + k] = a.f64[d * a.npad + o];
+        }
+        if (a.f32) {
+            for (int d = 0; d < 3; d++) a.f32b[d * a.npad + k] = a.f32[d * a.npad + o];
+        }
+        if (a.dem) {
+            a.omega2[k] = a.omega[o];
+            a.quat2[k] = a.quat[o];
+            if (a.t64)
+                for (int d = 0; d < 3; d++) a.t64b[d * a.npad + k] = a.t64[d * a.npad + o];
+            if (a.t32)
+                for (int d = 0; d < 3; d++) a.t32b[d * a.npad + k] = a.t32[d * a.npad + o];
+        }        BoxP box = a.box;
+        double gc = a.gc;
+        if (a.sysp) {
+            const SysP& S = a.sysp[a.psys[k]];
+            box = S.box;
+            gc = S.gc;
+        }
+        const double x[3] = {p.x, p.y, p.z};
+        int lf[3], hf[3];
+        image_flags(box, gc, x, lf, hf);
+        images =
+            uint32_t((1 + lf[0] + hf[0]) * (1 + lf[1] + hf[1]) * (1 + lf[2] + hf[2]) - 1);
+        a.gcnt[k] = images;
     }
-    if (i >= n) return;
-    if (sysp) {
-        const SysP& S = sysp[psys[i]];
-        box = S.box;
-        gc = S.gc;
+    // one atomic per tile that the wavefront's particles with images lie in
+    // (mostly one; counts of at most 26 are summed bit by bit)
+    const uint32_t tile = uint32_t(k >> kGhostTileLog2);
+    uint64_t left = __ballot(live && images != 0u);
+    while (left) {
+        const uint32_t t0 = __shfl(tile, __ffsll((unsigned long long)left) - 1, 64);
+        const bool mine = live && images != 0u && tile == t0;
+        uint32_t sum = 0u;
+#pragma unroll
+        for (int b = 0; b < 5; b++)
+            sum += uint32_t(__popcll(__ballot(mine && ((images >> b) & 1u)))) << b;
+        if ((threadIdx.x & 63u) == 0u) atomicAdd(&a.gtot[t0], sum);
+        left &= ~__ballot(mine);
     }
-    double4 p = pos[i];
-    double x[3] = {p.x, p.y, p.z};
-    int lf[3], hf[3];
-    image_flags(box, gc, x, lf, hf);
-    gcnt[i] = uint32_t((1 + lf[0] + hf[0]) * (1 + lf[1] + hf[1]) * (1 + lf[2] + hf[2]) - 1);
 }
 
-// periodic images of every particle (x shifted by exactly +-L per axis),
-// counted per bin cell for the image sort (cnt zeroed by k_ghost_count);
-// when they do not all fit, none is written and the live count is 0
-__global__ void k_ghost_emit(int64_t n, const double4* __restrict__ pos, BoxP box, double gc,
-                             GridP grid, const uint32_t* __restrict__ goff, int64_t ghost_cap,
-                             uint32_t* __restrict__ groot, uint8_t* __restrict__ gcode,
-                             double4* __restrict__ gpos, uint32_t* __restrict__ gkey,
-                             uint32_t* ng_live, Status* st, const SysP* __restrict__ sysp,
-                             const uint32_t* __restrict__ psys, uint32_t* __restrict__ cnt) {
-    int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-    const uint32_t total = goff[n];
+// periodic images of every particle (x shifted by exactly +-L per axis) in
+// particle order, counted per bin cell for the image sort; when they do not all
+// fit, none is written and the live count is 0. A block's first image follows
+// from the tiles' totals and the counts of its tile before it, so no scan of
+// the counts runs ahead.
+__global__ void __launch_bounds__(256) k_ghost_emit(
+    int64_t n, const double4* __restrict__ pos, BoxP box, double gc, GridP grid,
+    const uint32_t* __restrict__ gcnt, const uint32_t* __restrict__ gtot,
+    uint32_t* __restrict__ goff, int64_t ghost_cap, uint32_t* __restrict__ groot,
+    uint8_t* __restrict__ gcode, double4* __restrict__ gpos, uint32_t* __restrict__ gkey,
+    uint32_t* ng_live, Status* st, const SysP* __restrict__ sysp,
+    const uint32_t* __restrict__ psys, uint32_t* __restrict__ cnt) {
+    __shared__ uint32_t part[3][4];
+    const int lane = int(threadIdx.x & 63u), w = int(threadIdx.x >> 6);
+    const int64_t b0 = int64_t(blockIdx.x) * 256;
+    int64_t i = b0 + threadIdx.x;
+    const int64_t tile = b0 >> kGhostTileLog2, tiles = (n + (1 << kGhostTileLog2) - 1) >> kGhostTileLog2;
+    uint32_t before = 0u, total = 0u;
+    for (int64_t j = threadIdx.x; j < tiles; j += 256) {
+        const uint32_t t = gtot[j];
+        total += t;
+        if (j < tile) before += t;
+    }
+    for (int64_t j = (tile << kGhostTileLog2) + threadIdx.x; j < b0; j += 256) before += gcnt[j];
+    const uint32_t own = i < n ? gcnt[i] : 0u;
+    uint32_t incl = own;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        before += __shfl_xor(before, o, 64);
+        total += __shfl_xor(total, o, 64);
+    }
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t t = __shfl_up(incl, d, 64);
+        if (lane >= d) incl += t;
+    }
+    if (lane == 63) {
+        part[0][w] = before;
+        part[1][w] = total;
+        part[2][w] = incl;
+    }
+    __syncthreads();
+    uint32_t first = incl - own;
+    total = 0u;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        first += part[0][k] + (k < w ? part[2][k] : 0u);
+        total += part[1][k];
+    }
     const bool fits = int64_t(total) <= ghost_cap;
+    if (i < n) goff[i] = first;
     if (i == 0) {
+        goff[n] = total;
         st->ghost_total = total;
         *ng_live = fits ? total : 0u;
-        if (!fits) atomicOr(&st->overflow, 1u);
+        if (!fits) build_failed(st, 1u);
     }
     if (!fits) return;
     // every lane stays to the end: the per-cell counts are added once per
@@ -257,7 +353,7 @@ __global__ void k_ghost_emit(int64_t n, const double4* __restrict__ pos, BoxP bo
     double x[3] = {p.x, p.y, p.z};
     int lf[3], hf[3];
     image_flags(box, gc, x, lf, hf);
-    uint32_t g = live ? goff[i] : 0u;
+    uint32_t g = first;
     const int sv[3] = {0, 1, -1};
     for (int a = 0; a < 3; a++) {
         const int sx = sv[a];
@@ -284,7 +380,8 @@ __global__ void k_ghost_emit(int64_t n, const double4* __restrict__ pos, BoxP bo
                     gkey[g] = key;
                     g++;
                 }
-                // the image sort's per-cell count
+                // the image sort's per-cell count (one atomic per image instead of
+                // one per run of equal cells takes 4 us more at 4,000 atoms)
                 int h, t;
                 wave_runs(key, has, h, t);
                 if (has && int(threadIdx.x & 63) == t) atomicAdd(&cnt[key], uint32_t(t - h + 1));
@@ -293,19 +390,18 @@ __global__ void k_ghost_emit(int64_t n, const double4* __restrict__ pos, BoxP bo
     }
 }
 
-// combined bin starts: particles of a cell first (already sorted), then images
-
-// binned copies of position / neighbor skin radius and the encoded entry
+// binned copies of position / neighbor skin radius and the encoded entry:
+// particles of a cell first (already sorted), then its images
 __global__ void k_bin_fill(int64_t n, int64_t ghost_cap, const uint32_t* __restrict__ ng_live,
                            const uint32_t* __restrict__ key, const uint32_t* __restrict__ lstart,
                            const uint32_t* __restrict__ gstart,
                            const uint32_t* __restrict__ bstart,
-                           const uint32_t* __restrict__ gorder, const uint32_t* __restrict__ gkey,
+                           const uint32_t* __restrict__ placed, const uint32_t* __restrict__ gkey,
                            const double4* __restrict__ pos, const double* __restrict__ cutr,
                            const double4* __restrict__ gpos, const uint32_t* __restrict__ groot,
                            const uint8_t* __restrict__ gcode, double4* __restrict__ bin_pos,
                            uint32_t* __restrict__ bin_entry, uint32_t* __restrict__ bin_gidx,
-                           uint32_t* __restrict__ slot_local, uint32_t* __restrict__ bin_cell) {
+                           uint32_t* __restrict__ bin_cell) {
     const int64_t t = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
     if (t < n) {
         const uint32_t c = key[t];
@@ -313,15 +409,16 @@ __global__ void k_bin_fill(int64_t n, int64_t ghost_cap, const uint32_t* __restr
         const double4 p = pos[t];
         bin_pos[s] = make_double4(p.x, p.y, p.z, cutr[t]);
         bin_entry[s] = enc_entry(uint32_t(t), kCodeNone, false);
-        slot_local[t] = s;
         if (bin_cell) bin_cell[s] = c;
         return;
     }
     const int64_t gs = t - n;
     if (gs >= int64_t(*ng_live) || gs >= ghost_cap) return;
-    const uint32_t g = gorder[gs];
+    // images after the particles of a cell, in index order: bstart = lstart +
+    // gstart, so its first image's slot is bstart[c] + its particles
+    const uint32_t g = placed[gs];
     const uint32_t c = gkey[g];
-    const uint32_t s = bstart[c] + (lstart[c + 1] - lstart[c]) + (uint32_t(gs) - gstart[c]);
+    const uint32_t s = lstart[c + 1] + cell_rank(placed, gstart[c], gstart[c + 1], g);
     const double4 q = gpos[g];
     const uint32_t r = groot[g];
     bin_pos[s] = make_double4(q.x, q.y, q.z, cutr[r]);
@@ -504,7 +601,7 @@ __global__ void __launch_bounds__(256) k_build_tiles(CellArgs a) {
     tm.M = a.lstart[C + 1] - tm.s0;
     tm.G = uint32_t(tile_lanes(tm.M));
     tm.ginv = (65536u + tm.G - 1u) / tm.G;
-    if (total > 65535u) atomicOr(&a.st->overflow, 8u);  // tile index range
+    if (total > 65535u) build_failed(a.st, 8u);  // tile index range
     for (uint32_t ib = 0; ib < ni; ib += 64) {
         const uint32_t nib = ni - ib < 64u ? ni - ib : 64u;
         uint32_t cntv = 0, revv = 0;  // lane l: member ib + l
@@ -1076,69 +1173,44 @@ __global__ void __launch_bounds__(256) k_build_sparse(CellArgs a,
     }
 }
 
-// Row length of every particle: its own cell pass plus the pairs owned
-// through each of its periodic images. Row maxima go to per-block slots
-// (blk[2 b], blk[2 b + 1]); k_rows_gate reduces them, so no two blocks contend
-// for one address.
-__global__ void __launch_bounds__(256) k_row_totals(int64_t n, const uint32_t* __restrict__ goff,
-                                                    const uint32_t* __restrict__ ng_live,
-                                                    const uint32_t* __restrict__ gcnt,
-                                                    const uint32_t* __restrict__ nmain,
-                                                    const uint32_t* __restrict__ nhalf,
-                                                    uint32_t* __restrict__ nnb,
-                                                    uint32_t* __restrict__ blk,
-                                                    uint32_t* __restrict__ nx) {
-    __shared__ uint32_t lds[2][4];
-    const int64_t q = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-    uint32_t cnt = 0, nh = 0;
-    if (q < n) {
-        cnt = nmain[q];
-        nh = nhalf[q];
-        uint32_t xs = 0;
-        if (*ng_live != 0u)
-            for (uint32_t g = goff[q]; g < goff[q + 1]; g++) xs += gcnt[g];
-        cnt += xs;
-        nnb[q] = cnt;
-        if (nx) nx[q] = xs;  // tile rows: image-owned pairs kept apart
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const uint32_t x = __shfl_xor(cnt, o, 64), y = __shfl_xor(nh, o, 64);
-        cnt = x > cnt ? x : cnt;
-        nh = y > nh ? y : nh;
-    }
-    const int w = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) {
-        lds[0][w] = cnt;
-        lds[1][w] = nh;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t mc = 0, mh = 0;
-        for (int k = 0; k < int(blockDim.x >> 6); k++) {
-            mc = lds[0][k] > mc ? lds[0][k] : mc;
-            mh = lds[1][k] > mh ? lds[1][k] : mh;
-        }
-        blk[2 * blockIdx.x] = mc;
-        blk[2 * blockIdx.x + 1] = mh;
-    }
-}
-
-
-// Copy each image's scratch row to the end of its particle's row: after the
-// particle's own pass and the rows of the particle's earlier images.
+// The rows' ends, after the cell pass. Blocks of the first kind, a thread per
+// particle: the row length, its own cell pass plus the pairs owned through each
+// of its periodic images; a row that does not fit asks for rows of its length.
+// Blocks of the second, kCopyLanes threads per image: its scratch row copied to
+// the end of its particle's row, after the particle's own pass and the rows of
+// the particle's earlier images.
 constexpr int kCopyLanes = 16;
-__global__ void __launch_bounds__(256) k_copy_image_rows(int64_t ghost_cap, int64_t npad,
-                                                         int maxnb, int lg,
-                                                         const uint32_t* __restrict__ ng_live,
-                                                         const uint32_t* __restrict__ groot,
-                                                         const uint32_t* __restrict__ goff,
-                                                         const uint32_t* __restrict__ gcnt,
-                                                         const uint32_t* __restrict__ nmain,
-                                                         const uint32_t* __restrict__ gnbr,
-                                                         uint32_t* __restrict__ nbr,
-                                                         uint32_t* __restrict__ xnbr) {
-    const int64_t gt = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
+__global__ void __launch_bounds__(256) k_finish_rows(
+    int64_t n, int64_t nblocks, int64_t ghost_cap, int64_t npad, int maxnb, int lg,
+    const uint32_t* __restrict__ ng_live, const uint32_t* __restrict__ groot,
+    const uint32_t* __restrict__ goff, const uint32_t* __restrict__ gcnt,
+    const uint32_t* __restrict__ nmain, const uint32_t* __restrict__ gnbr,
+    uint32_t* __restrict__ nnb, uint32_t* __restrict__ nbr, uint32_t* __restrict__ nx,
+    uint32_t* __restrict__ xnbr, Status* st) {
+    if (int64_t(blockIdx.x) < nblocks) {
+        const int64_t q = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
+        uint32_t cnt = 0u;
+        if (q < n) {
+            uint32_t xs = 0u;
+            if (*ng_live != 0u)
+                for (uint32_t g = goff[q]; g < goff[q + 1]; g++) xs += gcnt[g];
+            cnt = nmain[q] + xs;
+            nnb[q] = cnt;
+            if (nx) nx[q] = xs;  // tile rows: image-owned pairs kept apart
+        }
+        if (__ballot(cnt > uint32_t(maxnb)) == 0ull) return;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            const uint32_t x = __shfl_xor(cnt, o, 64);
+            cnt = x > cnt ? x : cnt;
+        }
+        if ((threadIdx.x & 63u) == 0u) {
+            atomicMax(&st->max_row, int(cnt));
+            build_failed(st, 2u);
+        }
+        return;
+    }
+    const int64_t gt = (int64_t(blockIdx.x) - nblocks) * int64_t(blockDim.x) + threadIdx.x;
     const int64_t g = gt / kCopyLanes;
     const uint32_t t = uint32_t(gt % kCopyLanes);
     if (g >= ghost_cap || g >= int64_t(*ng_live)) return;
@@ -1361,7 +1433,7 @@ __global__ void k_hk_emit(int64_t n_old, int64_t npad_old, int maxnb_old, int lg
     if (p == 0) {
         const uint32_t total = off[n_old];
         st->hist_records = total;
-        if (total > cap) atomicOr(&st->overflow, 16u);
+        if (total > cap) build_failed(st, 16u);
     }
     if (p >= n_old) return;
     uint64_t m = cmask_old[p];
@@ -1492,45 +1564,6 @@ void neighbor_setup(Ctx& c);
 
 namespace {
 
-// End of a build attempt: row maxima from the per-block slots into the
-// status, and a build that did not fit stops the step sequence at `step`.
-__global__ void __launch_bounds__(256) k_rows_gate(int nblk, const uint32_t* __restrict__ blk,
-                                                   int maxnb, Status* st, int step) {
-    __shared__ uint32_t lds[2][4];
-    uint32_t mc = 0, mh = 0;
-    for (int b = threadIdx.x; b < nblk; b += blockDim.x) {
-        mc = blk[2 * b] > mc ? blk[2 * b] : mc;
-        mh = blk[2 * b + 1] > mh ? blk[2 * b + 1] : mh;
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const uint32_t x = __shfl_xor(mc, o, 64), y = __shfl_xor(mh, o, 64);
-        mc = x > mc ? x : mc;
-        mh = y > mh ? y : mh;
-    }
-    const int w = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) {
-        lds[0][w] = mc;
-        lds[1][w] = mh;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int k = 0; k < int(blockDim.x >> 6); k++) {
-            mc = lds[0][k] > mc ? lds[0][k] : mc;
-            mh = lds[1][k] > mh ? lds[1][k] : mh;
-        }
-        st->max_row = int(mc);
-        st->max_half = int(mh);
-        uint32_t ov = st->overflow;
-        if (mc > uint32_t(maxnb)) {
-            ov |= 2u;
-            st->overflow = ov;
-        }
-        // only the bits that make the host repeat the build (0-4) stop the step
-        if ((ov & 31u) != 0u && step < st->abort_step) st->abort_step = step;
-    }
-}
-
 
 void swap_alternates(Ctx& c);
 
@@ -1538,14 +1571,23 @@ void swap_alternates(Ctx& c);
 // alternates, record the build positions, then swap: the arrays are in the
 // new order and the alternates keep the previous one (tag2: the previous
 // tags, the source of the shear-history remap).
-void permute_all(Ctx& c, const uint32_t* order, int64_t n) {
+void permute_all(Ctx& c, bool placed, int64_t n) {
     const bool dem = c.model == 1;
     const bool mixed = c.precision == 1;
     PermArgs a;
     std::memset(&a, 0, sizeof(a));  // padding too: the bytes are a launch signature
     a.n = n;
     a.npad = c.npad;
-    a.order = order;
+    a.order = c.order.p;
+    a.order_out = c.order.p;
+    a.placed = c.placed.p;
+    a.start = c.start.p;
+    a.box = c.box;
+    a.gc = c.ghost_cutoff;
+    a.sysp = c.sysp_or_null();
+    a.psys = c.psys.p;
+    a.gcnt = c.gcnt.p;
+    a.gtot = c.gtot.p;
     // the source's arguments are the same whichever buffers hold the state:
     // c.third tells the kernel (Status::third)
     c.sorted_third = c.third;
@@ -1596,7 +1638,7 @@ void permute_all(Ctx& c, const uint32_t* order, int64_t n) {
         a.bxq = c.bxq.p;
         for (int d = 0; d < 3; d++) a.qs[d] = 4294967296.0 / c.box.L[d];
     }
-    launch(c, k_permute, blocks_for(n, 256), 256, a);
+    launch(c, placed ? k_permute<true> : k_permute<false>, blocks_for(n, 256), 256, a);
     MDD_HIP(hipGetLastError());
     swap_alternates(c);
     c.xq_valid = xq;
@@ -1628,10 +1670,22 @@ void swap_alternates(Ctx& c) {
     }
 }
 
+int64_t ghost_tiles(int64_t n) { return (n + (1 << kGhostTileLog2) - 1) >> kGhostTileLog2; }
+
+// The first kernel of a build, outside the recorded launches
+void launch_begin(Ctx& c, int step, bool retry) {
+    const int64_t ncells = c.grid.ncells;
+    c.cnt.resize(ncells);
+    c.gtot.resize(ghost_tiles(c.n));
+    k_rebuild_begin<<<std::min(blocks_for(ncells, 256), 512), 256, 0, c.stream>>>(
+        c.status.p, c.cnt.p, ncells, c.gtot.p, ghost_tiles(c.n), c.third ? 1 : 0, step,
+        retry ? 1 : 0);
+    MDD_HIP(hipGetLastError());
+}
+
 // pbc, spatial sort of the particles, and the previous list kept as the
 // source of the shear-history remap
 void rebuild_prepare(Ctx& c) {
-    if (!c.setup_done) neighbor_setup(c);
     c.xq_valid = false;  // the wrap moves particles
     const int64_t n = c.n;
     const int64_t ncells = c.grid.ncells;
@@ -1646,23 +1700,20 @@ void rebuild_prepare(Ctx& c) {
     c.gstart.resize(ncells + 1);
     c.gcnt.resize(n);
     c.goff.resize(n + 1);
+    c.gtot.resize(ghost_tiles(n));
     c.placed.resize(std::max<int64_t>(n, c.ghost_cap) + 1);
     // scan scratch sized once for every scan of this rebuild, so no buffer is
     // reallocated while kernels that use it are queued
     c.scan_tmp.resize(size_t((std::max<int64_t>(ncells, n) + 2047) / 2048 + 2));
-
-    // (launched by itself: its arguments differ from rebuild to rebuild)
-    k_rebuild_begin<<<blocks_for(ncells, 256) < 512 ? blocks_for(ncells, 256) : 512, 256, 0,
-                      c.stream>>>(c.status.p, c.cnt.p, ncells, c.third ? 1 : 0);
     // pbc + keys
     launch(c, k_wrap_key, blocks_for(n, 256), 256, n, c.third ? c.pos3.p : c.pos.p,
            c.third ? c.pos.p : c.pos3.p, c.image.p, c.box, c.grid, c.key.p, c.status.p,
            c.sysp_or_null(), c.psys.p, c.cnt.p);
-    // sort_atoms_by_bin: stable counting sort of particles by bin
-    counting_sort(c, c.key.p, n, nullptr, ncells, c.cnt.p, c.start.p, c.placed.p, c.order.p,
-                  nullptr, true, nullptr, nullptr, true);
-    // permute every particle array into the alternates, then swap
-    permute_all(c, c.order.p, n);
+    // sort_atoms_by_bin: stable counting sort of particles by bin, every
+    // particle array permuted into the alternates, then swapped
+    exclusive_scan(c, c.cnt.p, c.start.p, ncells);
+    place_by_key(c, c.key.p, n, nullptr, c.start.p, c.cnt.p, c.placed.p);
+    permute_all(c, true, n);
     // the previous list becomes the remap source
     c.remap_have_old = c.list_valid && dem;
     c.n_list_old = n;
@@ -1695,13 +1746,11 @@ void rebuild_attempt(Ctx& c) {
     c.ghost_code.resize(c.ghost_cap);
     c.ghost_pos.resize(c.ghost_cap);
     c.ghost_key.resize(c.ghost_cap + 1);  // last word: live image count
-    c.ghost_order.resize(c.ghost_cap);
     c.placed.resize(std::max<int64_t>(n, c.ghost_cap) + 1);
     const int64_t nall_max = n + c.ghost_cap;
     c.bin_pos.resize(nall_max);
     c.bin_entry.resize(nall_max);
     c.bin_gidx.resize(nall_max);
-    c.slot_of.resize(n);
     // sparse grids (fewer particles than cells): the per-member build kernel
     const bool sparse = c.nsys == 0 && !c.want_tile() &&
                         (c.build_mode == 2 || (c.build_mode == 0 && n < ncells));
@@ -1735,23 +1784,19 @@ void rebuild_attempt(Ctx& c) {
     uint32_t* ng_live = c.ghost_key.p + c.ghost_cap;
 
     // borders: periodic images and their bins
-    launch(c, k_ghost_count, blocks_for(n, 256), 256, n, c.pos.p, c.box, c.ghost_cutoff,
-                                                             c.gcnt.p, c.sysp_or_null(), c.psys.p,
-                                                             c.status.p, c.cnt.p, ncells);
-    exclusive_scan(c, c.gcnt.p, c.goff.p, n);
     launch(c, k_ghost_emit, blocks_for(n, 256), 256,
-        n, c.pos.p, c.box, c.ghost_cutoff, c.grid, c.goff.p, c.ghost_cap, c.ghost_root.p,
-        c.ghost_code.p, c.ghost_pos.p, c.ghost_key.p, ng_live, c.status.p, c.sysp_or_null(),
-        c.psys.p, c.cnt.p);
+        n, c.pos.p, c.box, c.ghost_cutoff, c.grid, c.gcnt.p, c.gtot.p, c.goff.p, c.ghost_cap,
+        c.ghost_root.p, c.ghost_code.p, c.ghost_pos.p, c.ghost_key.p, ng_live, c.status.p,
+        c.sysp_or_null(), c.psys.p, c.cnt.p);
     // images binned after the particles of each cell (bin_neighbor_list
     // steps 1-2b: counting sort in index order, images have the larger indices)
     // bin_start = particle start + image start of every cell, from the same scan
-    counting_sort(c, c.ghost_key.p, c.ghost_cap, ng_live, ncells, c.cnt.p, c.gstart.p, c.placed.p,
-                  c.ghost_order.p, nullptr, true, c.start.p, c.bin_start.p, true);
+    exclusive_scan(c, c.cnt.p, c.gstart.p, ncells, c.start.p, c.bin_start.p);
+    place_by_key(c, c.ghost_key.p, c.ghost_cap, ng_live, c.gstart.p, c.cnt.p, c.placed.p);
     launch(c, k_bin_fill, blocks_for(nall_max, 256), 256,
-        n, c.ghost_cap, ng_live, c.key.p, c.start.p, c.gstart.p, c.bin_start.p, c.ghost_order.p,
+        n, c.ghost_cap, ng_live, c.key.p, c.start.p, c.gstart.p, c.bin_start.p, c.placed.p,
         c.ghost_key.p, c.pos.p, c.cutr.p, c.ghost_pos.p, c.ghost_root.p, c.ghost_code.p,
-        c.bin_pos.p, c.bin_entry.p, c.bin_gidx.p, c.slot_of.p, sparse ? c.bin_cell.p : nullptr);
+        c.bin_pos.p, c.bin_entry.p, c.bin_gidx.p, sparse ? c.bin_cell.p : nullptr);
     // rows: one wavefront per cell (or one lane per member on sparse grids),
     // then image-owned pairs appended
     CellArgs ca;
@@ -1821,14 +1866,10 @@ void rebuild_attempt(Ctx& c) {
             launch(c, k_build_rows<false, false, 10>, rblocks, 256, ca, wl);
     }
     const int tblocks = blocks_for(n, 256);
-    c.row_blk.resize(size_t(2) * tblocks);
-    launch(c, k_row_totals, tblocks, 256, n, c.goff.p, ng_live, c.gcnt_img.p, c.nmain.p,
-                                                c.nhalf.p, c.nnb.p, c.row_blk.p,
-                                                tile ? c.nx.p : nullptr);
-    c.row_nblk = tblocks;
-    launch(c, k_copy_image_rows, blocks_for(c.ghost_cap * kCopyLanes, 256), 256,
-        c.ghost_cap, c.npad, c.maxnb, c.lg, ng_live, c.ghost_root.p, c.goff.p, c.gcnt_img.p,
-        c.nmain.p, c.gnbr.p, c.nbr.p, tile ? c.xnbr.p : nullptr);
+    launch(c, k_finish_rows, tblocks + blocks_for(c.ghost_cap * kCopyLanes, 256), 256, n,
+           int64_t(tblocks), c.ghost_cap, c.npad, c.maxnb, c.lg, ng_live, c.ghost_root.p, c.goff.p,
+           c.gcnt_img.p, c.nmain.p, c.gnbr.p, c.nnb.p, c.nbr.p, tile ? c.nx.p : nullptr,
+           tile ? c.xnbr.p : nullptr, c.status.p);
     MDD_HIP(hipGetLastError());
     c.list_tile = tile;
     if (dem && c.remap_sorted && c.remap_have_old) {
@@ -1996,7 +2037,9 @@ void remove_outside(Ctx& c) {
     if (c.sorted_third) swap_state(c);
     h2d(c, c.order.p, fin.data(), sizeof(uint32_t) * size_t(len));
     h2d(c, c.start.p, start.data(), sizeof(uint32_t) * (size_t(ncells) + 1));
-    permute_all(c, c.order.p, len);
+    c.gtot.resize(ghost_tiles(len));
+    fill_u32(c, c.gtot.p, 0u, ghost_tiles(len));
+    permute_all(c, false, len);
     k_clear_exit<<<1, 1, 0, c.stream>>>(c.status.p);
     MDD_HIP(hipGetLastError());
     MDD_HIP(hipStreamSynchronize(c.stream));
@@ -2006,12 +2049,14 @@ void remove_outside(Ctx& c) {
 
 // full rebuild, checked on the host before it returns
 void rebuild(Ctx& c) {
+    if (!c.setup_done) neighbor_setup(c);
+    launch_begin(c, INT_MAX, false);
     rebuild_prepare(c);
-    bool fitted = false;
+    bool fitted = false, again = false;
     for (int attempt = 0; attempt < 6 && !fitted; attempt++) {
+        if (again) launch_begin(c, INT_MAX, true);
+        again = true;
         rebuild_attempt(c);
-        k_rows_gate<<<1, 256, 0, c.stream>>>(c.row_nblk, c.row_blk.p, c.maxnb, c.status.p,
-                                             INT_MAX);
         MDD_HIP(hipMemcpyAsync(c.status_host, c.status.p, sizeof(Status), hipMemcpyDeviceToHost,
                                c.stream));
         MDD_HIP(hipStreamSynchronize(c.stream));
@@ -2094,7 +2139,7 @@ void release_graphs(Ctx& c) {
 }
 
 // One rebuild. A first attempt (not a retry) is recorded and issued as a
-// graph: its ~30 launches reach the device at once instead of one host
+// graph: its launches (10 for LJ) reach the device at once instead of one host
 // launch at a time.
 void launch_sort_check(Ctx& c, int step) {
     if (c.n < 2) return;
@@ -2111,6 +2156,8 @@ void rebuild_async(Ctx& c, int step, bool retry) {
         if (c.rb_chunk_mark) std::swap(c.rb_ev[3 * c.rb_pending], c.rb_mark);
     }
     c.rb_chunk_mark = false;
+    if (!retry && !c.setup_done) neighbor_setup(c);
+    launch_begin(c, step, retry);
     const bool record = !retry && c.graphs_on && c.setup_done;
     if (record) {
         c.rec.sig.clear();
@@ -2141,8 +2188,6 @@ void rebuild_async(Ctx& c, int step, bool retry) {
             c.rec.frees.clear();
         }
     }
-    k_rows_gate<<<1, 256, 0, c.stream>>>(c.row_nblk, c.row_blk.p, c.maxnb, c.status.p, step);
-    MDD_HIP(hipGetLastError());
     if (timed) MDD_HIP(hipEventRecord(c.rb_ev[3 * c.rb_pending++ + 2], c.stream));
 }
 
