@@ -1207,9 +1207,21 @@ struct Sums {
     }
 };
 
-template <typename R>
+// Workgroup sizes of the DEM pair passes, whose wavefronts take unequal time
+// (rows and contacts differ) and hold 3 places per SIMD: a workgroup's places
+// are free for the next one only when its last wavefront ends. In us per step
+// with workgroups of 256, 128 and 64: a bed of 250,000 (double precision, two
+// lanes) 64.4, 63.2, 62.7; of 140,000 with adhesion (four lanes) 65.1, 64.1,
+// 63.5; of 4,000,000 (queued contacts) 910, 900, 893; a gas of 200,000 (one
+// lane, short rows) 17.9, 17.4, 19.1.
+__host__ __device__ constexpr int hertz_block(int lg, bool quad) {
+    return !quad ? 256 : (lg == 0 ? 128 : 64);
+}
+constexpr int kWaveBlock = 64, kExtBlock = 64;
+
+template <typename R, int N>
 struct SumSlot {
-    R v[6][256];
+    R v[6][N];
     __device__ inline void put(const Sums<R>& s) {
         const int t = int(threadIdx.x);
         v[0][t] = s.fx;
@@ -1238,8 +1250,8 @@ struct RowSums {
     Sums<R> cur;
     int cls = 0;
     unsigned have = 0;  // bit c: class c has contacts
-    __device__ inline SumSlot<R>* slots() const {
-        __shared__ SumSlot<R> s[!QUAD ? 1 : (LG == 1 ? 1 : 4)];
+    __device__ inline auto* slots() const {
+        __shared__ SumSlot<R, hertz_block(LG, QUAD)> s[!QUAD ? 1 : (LG == 1 ? 1 : 4)];
         return s;
     }
     // the next contact is entry k
@@ -1384,7 +1396,7 @@ __device__ inline void hertz_particle(const ForceArgs& a, const S& s, int64_t i,
 // band of bin columns, so the partners it gathers stay in its L2), or null
 // for the particles in index order
 template <typename R, int LG, bool VIR, bool QUAD, typename S>
-__global__ void __launch_bounds__(256, 3) k_hertz(ForceArgs a, S s, const uint32_t* __restrict__ order) {
+__global__ void __launch_bounds__(hertz_block(LG, QUAD), 3) k_hertz(ForceArgs a, S s, const uint32_t* __restrict__ order) {
     constexpr int G = 1 << LG;
     // XCD-aware block order: each XCD's L2 holds the positions of one
     // contiguous (spatially sorted) range of particles and its neighbors
@@ -1475,9 +1487,9 @@ __device__ inline void wave_contacts(const ForceArgs& a, WaveQueue& q, int nq, u
 // order: tile order (particle order[k] for k < n), or null for XCD-aware
 // block order over the particles
 template <typename R, typename S>
-__global__ void __launch_bounds__(256) k_hertz_wave(ForceArgs a, S s,
+__global__ void __launch_bounds__(kWaveBlock) k_hertz_wave(ForceArgs a, S s,
                                                     const uint32_t* __restrict__ order) {
-    __shared__ WaveQueue queues[4];
+    __shared__ WaveQueue queues[kWaveBlock / 64];
     WaveQueue& q = queues[threadIdx.x >> 6];
     const int lane = int(threadIdx.x & 63);
     if (gated(a)) return;
@@ -1625,8 +1637,12 @@ __global__ void __launch_bounds__(256) k_hertz_unlisted(ForceArgs a, S s) {
 // 0-2, rolling 3-5, twist 6, canonical sign). Every pair quantity is FP64;
 // only the sums are kept in R. Pairs are evaluated in the owner frame as in
 // k_hertz, so both rows of a pair carry the same history.
+//
+// A chain of gathers and 64-bit roots and quotients per pair: wavefronts in
+// flight hide it. Held to the registers of 3 per SIMD (170 left 2), a step of a
+// bed of 140,000 takes 65 us instead of 79; at 4 (128 registers) it spills: 127.
 template <typename R, int LG, typename S>
-__global__ void __launch_bounds__(256) k_contact_ext(ForceArgs a, S s) {
+__global__ void __launch_bounds__(kExtBlock, 3) k_contact_ext(ForceArgs a, S s) {
     constexpr int G = 1 << LG;
     // XCD-aware block order: each XCD's L2 holds the positions of one
     // contiguous (spatially sorted) range of particles and its neighbors
@@ -2010,11 +2026,12 @@ ForceArgs make_args(Ctx& c, int step) {
 // given, are attached to the dispatch itself (hipExtLaunchKernelGGL), so
 // they time the kernel alone, as a kernel trace does.
 template <typename K, typename... A>
-void launch_force_kernel(Ctx& c, K kern, int nb, hipEvent_t e0, hipEvent_t e1, const A&... args) {
+void launch_force_kernel(Ctx& c, K kern, int nb, int threads, hipEvent_t e0, hipEvent_t e1,
+                         const A&... args) {
     if (e0)
-        hipExtLaunchKernelGGL(kern, dim3(nb), dim3(256), 0, c.stream, e0, e1, 0, args...);
+        hipExtLaunchKernelGGL(kern, dim3(nb), dim3(threads), 0, c.stream, e0, e1, 0, args...);
     else
-        kern<<<nb, 256, 0, c.stream>>>(args...);
+        kern<<<nb, threads, 0, c.stream>>>(args...);
 }
 
 // fixed-point positions of every particle (x * qs per axis, modulo 2^32)
@@ -2051,10 +2068,10 @@ void launch_lj(Ctx& c, const ForceArgs& a, const S& s, hipEvent_t e0, hipEvent_t
     const int64_t threads = c.n << c.list_lg;
     const int nb = blocks_for(threads, 256);
     switch (c.list_lg) {
-        case 0: launch_force_kernel(c, k_lj<R, E, 0, S>, nb, e0, e1, a, s); break;
-        case 1: launch_force_kernel(c, k_lj<R, E, 1, S>, nb, e0, e1, a, s); break;
-        case 3: launch_force_kernel(c, k_lj<R, E, 3, S>, nb, e0, e1, a, s); break;
-        default: launch_force_kernel(c, k_lj<R, E, 2, S>, nb, e0, e1, a, s); break;
+        case 0: launch_force_kernel(c, k_lj<R, E, 0, S>, nb, 256, e0, e1, a, s); break;
+        case 1: launch_force_kernel(c, k_lj<R, E, 1, S>, nb, 256, e0, e1, a, s); break;
+        case 3: launch_force_kernel(c, k_lj<R, E, 3, S>, nb, 256, e0, e1, a, s); break;
+        default: launch_force_kernel(c, k_lj<R, E, 2, S>, nb, 256, e0, e1, a, s); break;
     }
 }
 
@@ -2094,24 +2111,25 @@ bool launch_lj_post(Ctx& c, const ForceArgs& a0, hipEvent_t e0, hipEvent_t e1, i
 
 template <typename R, bool VIR, typename S>
 void launch_hertz(Ctx& c, const ForceArgs& a, const S& s, hipEvent_t e0, hipEvent_t e1) {
-    auto go = [&](int lanes_log2, auto kern, auto... more) {
-        launch_force_kernel(c, kern, blocks_for(c.n << lanes_log2, 256), e0, e1, a, s, more...);
+    auto go = [&](int block, int lanes_log2, auto kern, auto... more) {
+        launch_force_kernel(c, kern, blocks_for(c.n << lanes_log2, block), block, e0, e1, a, s,
+                            more...);
     };
     const bool pick = c.lanes_auto;
     const int lg = pick ? 2 : c.list_lanes;
     if (c.ext_on) {
         switch (lg) {
-            case 0: go(0, k_contact_ext<R, 0, S>); break;
-            case 1: go(1, k_contact_ext<R, 1, S>); break;
-            case 3: go(3, k_contact_ext<R, 3, S>); break;
-            default: go(2, k_contact_ext<R, 2, S>); break;
+            case 0: go(kExtBlock, 0, k_contact_ext<R, 0, S>); break;
+            case 1: go(kExtBlock, 1, k_contact_ext<R, 1, S>); break;
+            case 3: go(kExtBlock, 3, k_contact_ext<R, 3, S>); break;
+            default: go(kExtBlock, 2, k_contact_ext<R, 2, S>); break;
         }
         return;
     }
     const bool tiles = c.tile_order && c.tile_ok && c.nsys == 0;
     const uint32_t* ord = tiles ? static_cast<const uint32_t*>(c.tile_list.p) : nullptr;
     if (c.dem_wave && !pick && lg == 0 && !VIR) {
-        go(0, k_hertz_wave<R, S>, ord);
+        go(kWaveBlock, 0, k_hertz_wave<R, S>, ord);
         return;
     }
     if constexpr (!VIR) {
@@ -2124,17 +2142,18 @@ void launch_hertz(Ctx& c, const ForceArgs& a, const S& s, hipEvent_t e0, hipEven
             // of 20,000 29 / 23. Tile order pays on full rows only (a gas of
             // 200,000: 17.9 us with it, 17.0 without).
             if (c.n >= 65536 && 10 * int64_t(c.status_host->listed) < 9 * c.n)
-                go(0, k_hertz<R, 0, false, true, S>, static_cast<const uint32_t*>(nullptr));
+                go(hertz_block(0, true), 0, k_hertz<R, 0, false, true, S>,
+                   static_cast<const uint32_t*>(nullptr));
             else
-                go(1, k_hertz<R, 1, false, true, S>, ord);
+                go(hertz_block(1, true), 1, k_hertz<R, 1, false, true, S>, ord);
             return;
         }
     }
     switch (lg) {
-        case 0: go(0, k_hertz<R, 0, VIR, false, S>, ord); break;
-        case 1: go(1, k_hertz<R, 1, VIR, false, S>, ord); break;
-        case 3: go(3, k_hertz<R, 3, VIR, false, S>, ord); break;
-        default: go(2, k_hertz<R, 2, VIR, false, S>, ord); break;
+        case 0: go(256, 0, k_hertz<R, 0, VIR, false, S>, ord); break;
+        case 1: go(256, 1, k_hertz<R, 1, VIR, false, S>, ord); break;
+        case 3: go(256, 3, k_hertz<R, 3, VIR, false, S>, ord); break;
+        default: go(256, 2, k_hertz<R, 2, VIR, false, S>, ord); break;
     }
 }
 
