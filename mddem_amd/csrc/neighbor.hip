@@ -743,7 +743,7 @@ struct RowStage {
     uint32_t ent[NCH * 64];  // bin slots, then entries, of the candidates
 };
 // four blocks (16 wavefronts) share a CU's 160 KB
-static_assert(kCellWaves * sizeof(RowStage<10>) * 4 <= 160 * 1024, "four blocks per CU");
+static_assert(kCellWaves * sizeof(RowStage<11>) * 4 <= 160 * 1024, "four blocks per CU");
 
 // Append f of the lanes in `pass` (wavefront-uniform) to the list whose end is
 // the LDS byte address `at` (uniform), which advances. Written as one block
@@ -1850,16 +1850,19 @@ void rebuild_attempt(Ctx& c) {
         ca.inner_blocks = uint32_t(blocks_for(ca.inner_cells << wl, kCellWaves));
         const int rblocks = int(ca.inner_blocks) +
                             int((((2 * ca.inner_first) << wl) + kCellWaves - 1) / kCellWaves);
-        // candidates of a cell at the mean density, with a tenth to spare: 640
-        // fit 10 chunks at 4 wavefronts per SIMD (LJ fluids: 490 to 600); the
-        // wider bins of a box of few cells need 16, at 3 wavefronts (4,000
-        // atoms: 5 bins a side, 860 candidates; from memory instead of
-        // registers such a build takes 58 us instead of 35)
+        // candidates of a cell at the mean density, with 4% to spare (a liquid's
+        // fluctuate by 1 to 2%; a cell beyond the chunks reads them from memory
+        // for each batch of members): 11 chunks of 64 is what 4 wavefronts per
+        // SIMD leave registers for, and enough for LJ fluids from 20,000 atoms
+        // on (490 to 680). With 10, whole rebuilds took 126 us instead of 105
+        // at 49,000 atoms, 231 instead of 208 at 256,000. The wider bins of a
+        // box of few cells need 16, at 3 wavefronts (4,000 atoms: 5 bins a
+        // side, 860 candidates; from memory their build takes 58 us, not 35).
         const double cand = double(n) / c.bins_in_box * double(c.full.size());
         if (c.nsys > 0)
             launch(c, k_build_rows<false, true, 10>, rblocks, 256, ca, wl);
-        else if (c.uniform && cand * 1.1 <= 640.0)
-            launch(c, k_build_rows<true, false, 10>, rblocks, 256, ca, wl);
+        else if (c.uniform && cand * 1.04 <= 704.0)
+            launch(c, k_build_rows<true, false, 11>, rblocks, 256, ca, wl);
         else if (c.uniform)
             launch(c, k_build_rows<true, false, 16>, rblocks, 256, ca, wl);
         else
