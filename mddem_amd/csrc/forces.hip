@@ -151,6 +151,32 @@ struct alignas(16) ShiftPair {
     double j[3], i[3], pad[2];
 };
 
+// What a lane's walk of a mixed LJ row starts from
+template <int LG>
+struct LjHead {
+    int4 qi;
+    int cnt;
+    uint32_t en[MDD_LJ_BATCH];
+};
+
+// (no load depends on another, the row's first entries included, which are read
+// whether or not the row is as long: one memory latency, together with the
+// launch's gate. A step of 32,000 atoms 28.2 -> 27.2 us, of 256,000, where other
+// wavefronts hide it, 66.9 -> 66.5; the 64-bit pass, with twice the registers
+// in it, gained nothing at 32,000 and lost 1% at 4,000.)
+template <int LG>
+__device__ inline LjHead<LG> lj_head(const ForceArgs& a, int64_t i, int t) {
+    LjHead<LG> h;
+    h.qi = a.xq[i];
+    h.cnt = int(a.nnb[i]);
+#pragma unroll
+    for (int u = 0; u < MDD_LJ_BATCH; u++)
+        h.en[u] = ((u + 1) << LG) <= a.maxnb
+                      ? (a.nbr + u * (a.npad << LG))[(uint32_t(i) << LG) + uint32_t(t)]
+                      : 0u;
+    return h;
+}
+
 // Mixed LJ row of particle i (lane t of G) on fixed-point positions: one
 // 16-byte gather per neighbor; the 32-bit coordinate differences are the
 // minimum-image separation in units of L / 2^32, so image entries need no
@@ -162,14 +188,14 @@ struct alignas(16) ShiftPair {
 // for the cutoff's neighborhood at once: 83 vector instructions per 3 pairs
 // instead of 93, 26.6 us with the final half step.
 template <int LG>
-__device__ inline void lj_row_fixed_force(const ForceArgs& a, int64_t i, int t, float& fx_out,
-                                          float& fy_out, float& fz_out) {
+__device__ inline void lj_row_fixed_force(const ForceArgs& a, const LjHead<LG>& h, int64_t i,
+                                          int t, float& fx_out, float& fy_out, float& fz_out) {
     constexpr int G = 1 << LG;
     constexpr int kB = MDD_LJ_BATCH;
-    int cnt = int(a.nnb[i]);
+    int cnt = h.cnt;
     if (cnt > a.maxnb) cnt = a.maxnb;
     const int64_t stride = a.npad << LG;
-    const int4 qi = a.xq[i];
+    const int4 qi = h.qi;
     const float sx = a.qf[0], sy = a.qf[1], sz = a.qf[2];
     const float cut2 = float(a.cut2), lj1 = float(a.lj1), lj2 = float(a.lj2);
     const float cut2_eps = 1e-6f * cut2;
@@ -208,7 +234,7 @@ __device__ inline void lj_row_fixed_force(const ForceArgs& a, int64_t i, int t, 
     const uint32_t* rows = a.nbr;
     uint32_t en[kB];
 #pragma unroll
-    for (int u = 0; u < kB; u++) en[u] = u < own ? (rows + u * stride)[lane_at] : 0u;
+    for (int u = 0; u < kB; u++) en[u] = u < own ? h.en[u] : 0u;
     // the batch of kB entries from m on, while the next one's are loaded.
     // WHOLE: both are whole in every lane's row
     auto batch = [&](int m, auto whole) {
@@ -251,9 +277,10 @@ __device__ inline void begin_step(const ForceArgs& a, const S& s) {
 }
 
 template <int LG, typename S>
-__device__ inline void lj_row_fixed(const ForceArgs& a, const S& s, int64_t i, int t) {
+__device__ inline void lj_row_fixed(const ForceArgs& a, const S& s, const LjHead<LG>& h, int64_t i,
+                                    int t) {
     float fx, fy, fz;
-    lj_row_fixed_force<LG>(a, i, t, fx, fy, fz);
+    lj_row_fixed_force<LG>(a, h, i, t, fx, fy, fz);
     if (t != 0) return;
     if constexpr (std::is_same<S, StepArgs>::value) {
         step_advance(s, i, a.pos[i], step_load(s, i), double(fx), double(fy), double(fz), 0.0, 0.0, 0.0);
@@ -284,15 +311,21 @@ __global__ void __launch_bounds__(256 << LG) k_lj_post(ForceArgs a, PostArgs p) 
     constexpr int G = 1 << LG;
     __shared__ double ke_lds[256];
     __shared__ double lds4[4];
-    if (gated(a)) return;
     const int64_t pb = xcd_block(blockIdx.x, gridDim.x);
     const int local = int(threadIdx.x >> LG);
     const int t = int(threadIdx.x & (G - 1));
     const int64_t i = pb * 256 + local;
     double ke = 0.0;
-    if (i < a.n) {
+    const bool live = i < a.n;
+    const int stop = a.st->abort_step;
+    const LjHead<LG> h = lj_head<LG>(a, live ? i : 0, t);
+    // (keeps the compiler from sinking the loads below the gate)
+    __asm__ volatile("" ::"v"(stop), "v"(h.qi.x), "v"(h.cnt), "v"(h.en[0]),
+                     "v"(h.en[MDD_LJ_BATCH - 1]));
+    if (a.step >= 0 && stop <= a.step) return;
+    if (live) {
         float fx, fy, fz;
-        lj_row_fixed_force<LG>(a, i, t, fx, fy, fz);
+        lj_row_fixed_force<LG>(a, h, i, t, fx, fy, fz);
         if (t == 0) {
             a.f32[i] = fx;
             a.f32[a.npad + i] = fy;
@@ -361,16 +394,23 @@ __global__ void __launch_bounds__(256) k_lj(ForceArgs a, S s) {
         q.pad[0] = q.pad[1] = 0.0;
         shp[threadIdx.x] = q;
     }
+    if constexpr (sizeof(R) == 4 && !ENERGY) {
+        if (a.xq) {
+            const int stop = a.st->abort_step;
+            const LjHead<LG> h = lj_head<LG>(a, i < a.n ? i : 0, t);
+            // (keeps the compiler from sinking the loads below the gate)
+            __asm__ volatile("" ::"v"(stop), "v"(h.qi.x), "v"(h.cnt), "v"(h.en[0]),
+                             "v"(h.en[MDD_LJ_BATCH - 1]));
+            if (i >= a.n || (a.step >= 0 && stop <= a.step)) return;
+            begin_step(a, s);
+            lj_row_fixed<LG>(a, s, h, i, t);
+            return;
+        }
+    }
     __syncthreads();
     if (i >= a.n) return;
     if (gated(a)) return;
     begin_step(a, s);
-    if constexpr (sizeof(R) == 4 && !ENERGY) {
-        if (a.xq) {
-            lj_row_fixed<LG>(a, s, i, t);
-            return;
-        }
-    }
     const double4 xi = a.pos[i];
     int cnt = int(a.nnb[i]);
     if (cnt > a.maxnb) cnt = a.maxnb;
@@ -1316,24 +1356,47 @@ struct RowSums {
     }
 };
 
-template <typename R, int LG, bool VIR, bool QUAD, typename S>
-__device__ inline void hertz_particle(const ForceArgs& a, const S& s, int64_t i, int t) {
+// What a lane's walk of its row starts from. None of it depends on another
+// load, the row's first entries included (read whether or not the row is as
+// long), so it costs one memory latency, together with the launch's gate: a
+// step of a gas of 500 spheres 6.85 -> 6.4 us, of 200,000 16.6 -> 15.9, of an
+// ensemble of 282,000 19.2 -> 18.7.
+struct RowHead {
+    double4 pi;
+    uint32_t ti, e0, e1, e2;
+    int cnt;
+};
+
+template <int LG, bool QUAD>
+__device__ inline RowHead row_head(const ForceArgs& a, int64_t i, int t) {
+    constexpr bool kPair = QUAD && LG == 1;  // the second entry is t + 4 or t + 2
+    RowHead h;
+    h.pi = a.pos[i];
+    h.ti = a.type[i];
+    h.cnt = 0;
+    h.e0 = h.e1 = h.e2 = 0u;
+    if (a.use_pairs) {
+        auto raw = [&](int k) { return k < a.maxnb ? a.nbr[row_addr(i, k, a.npad, a.rl)] : 0u; };
+        h.cnt = int(a.nnb[i]);
+        h.e0 = raw(t);
+        h.e1 = raw(t + (kPair ? 4 : 1 << LG));
+        if (kPair) h.e2 = raw(t + 2);
+    }
+    return h;
+}
+
+template <typename R, int LG, bool VIR, bool QUAD, bool EARLY, typename S>
+__device__ inline void hertz_particle(const ForceArgs& a, const S& s, int64_t i, int t,
+                                      const RowHead& head, Pre<S> pre) {
     constexpr int G = 1 << LG;
-    const double4 pi = a.pos[i];
-    const uint32_t ti = a.type[i];
-    // a single system at one lane in FP32 has registers to load the
-    // integration's inputs before the row is walked (200,000 gas spheres: 18.3
-    // -> 17.5 us a step; in a batched ensemble, whose per-system lookups are
-    // the longer chain, 19.6 -> 21.4 us, so not there)
-    constexpr bool kEarly = LG == 0 && QUAD && sizeof(R) == 4;
-    Pre<S> pre;
-    if (kEarly) pre = preload(s, i);
+    const double4 pi = head.pi;
+    const uint32_t ti = head.ti;
     double Lx, Ly, Lz;
     const SysP* sys = particle_box(a, i, Lx, Ly, Lz);
     RowSums<R, LG, QUAD> sum;
     double w0 = 0.0, w1 = 0.0, w2 = 0.0, w3 = 0.0, w4 = 0.0, w5 = 0.0;
     if (a.use_pairs) {
-        int cnt = int(a.nnb[i]);
+        int cnt = head.cnt;
         if (cnt > a.maxnb) cnt = a.maxnb;
         // contact bits only ever cover row slots: an empty row has none, so
         // a particle without neighbors reads and writes no contact state
@@ -1353,7 +1416,8 @@ __device__ inline void hertz_particle(const ForceArgs& a, const S& s, int64_t i,
         // particle 0 and are not used); the partner's velocity and spin are
         // read only for pairs in contact, so they are not fetched ahead
         int k = t, kn = after(t);
-        uint32_t e_n = entry(k), e_nn = entry(kn);
+        uint32_t e_n = k < cnt ? head.e0 : 0u;
+        uint32_t e_nn = kn < cnt ? (QUAD && LG == 1 && kn == t + 2 ? head.e2 : head.e1) : 0u;
         double4 pj_n = a.pos[entry_idx(e_n)];
         while (k < cnt) {
             const uint32_t e = e_n;
@@ -1415,7 +1479,7 @@ __device__ inline void hertz_particle(const ForceArgs& a, const S& s, int64_t i,
         a.vir[4 * np + i] = w4;
         a.vir[5 * np + i] = w5;
     }
-    if (!kEarly) pre = preload(s, i);
+    if (!EARLY) pre = preload(s, i);
     finish_particle<R>(a, s, i, pi, pre, ti, sum.cur.fx, sum.cur.fy, sum.cur.fz, sum.cur.tx,
                        sum.cur.ty, sum.cur.tz);
 }
@@ -1432,9 +1496,27 @@ __global__ void __launch_bounds__(hertz_block(LG, QUAD), 3) k_hertz(ForceArgs a,
     const int64_t k = gt >> LG;
     const int t = int(gt & (G - 1));
     if (k >= a.n) return;
-    if (gated(a)) return;
+    // a single system at one lane in FP32 has registers to load the
+    // integration's inputs before the row is walked (200,000 gas spheres: 18.3
+    // -> 17.5 us a step; in a batched ensemble, whose per-system lookups are
+    // the longer chain, 19.6 -> 21.4 us, so not there; nor at two lanes, where
+    // they leave 2 wavefronts per SIMD: 20,000 spheres 7.0 -> 7.5 us)
+    constexpr bool EARLY = LG == 0 && QUAD && sizeof(R) == 4;
+    const int64_t i = order ? int64_t(order[k]) : k;
+    const int stop = a.st->abort_step;
+    const RowHead h = row_head<LG, QUAD>(a, i, t);
+    Pre<S> pre;
+    if (EARLY) pre = preload(s, i);
+    // (an empty statement that takes the loaded values keeps the compiler
+    // from sinking their loads below the gate)
+    __asm__ volatile("" ::"v"(stop), "v"(h.pi.x), "v"(h.pi.w), "v"(h.ti), "v"(h.cnt), "v"(h.e0),
+                     "v"(h.e1), "v"(h.e2));
+    if constexpr (EARLY && std::is_same<S, StepArgs>::value)
+        __asm__ volatile("" ::"v"(pre.in.v.x), "v"(pre.in.v.w), "v"(pre.in.w.x), "v"(pre.in.w.w),
+                         "v"(pre.in.b.x), "v"(pre.in.b.z));
+    if (a.step >= 0 && stop <= a.step) return;
     begin_step(a, s);
-    hertz_particle<R, LG, VIR, QUAD>(a, s, order ? int64_t(order[k]) : k, t);
+    hertz_particle<R, LG, VIR, QUAD, EARLY>(a, s, i, t, h, pre);
 }
 
 // The same pass with the pairs in contact compacted per wavefront (one lane
@@ -1622,8 +1704,11 @@ __global__ void __launch_bounds__(256) k_hertz_listed(ForceArgs a, S s) {
     begin_step(a, s);
     const uint32_t nl = *a.listed_n;
     const uint32_t stride = gridDim.x * blockDim.x;
-    for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < nl; k += stride)
-        hertz_particle<R, 0, false, false>(a, s, int64_t(a.listed[k]), 0);
+    for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < nl; k += stride) {
+        const int64_t i = int64_t(a.listed[k]);
+        hertz_particle<R, 0, false, false, false>(a, s, i, 0, row_head<0, false>(a, i, 0),
+                                                  Pre<S>());
+    }
 }
 
 template <typename R, typename S>
