@@ -42,29 +42,18 @@ __device__ inline void wave_lds_sync() {
 }
 
 // Runs of equal keys inside a wavefront: the lane of the run head (h) and
-// of the run tail (t). Invalid lanes form runs of their own.
+// of the run tail (t). Invalid lanes form runs of their own. From the ballot of
+// the heads: as two scans of shuffles it was most of the image pass at 4,000 atoms
+// (8.2 -> 6.3 us; 10.1 -> 8.0 at 256,000).
 __device__ inline void wave_runs(uint32_t key, bool valid, int& h, int& t) {
     const int lane = threadIdx.x & 63;
     const uint32_t kp = __shfl_up(key, 1, 64);
-    const int vp = __shfl_up(int(valid), 1, 64);
-    const uint32_t kn = __shfl_down(key, 1, 64);
-    const int vn = __shfl_down(int(valid), 1, 64);
-    const bool head = lane == 0 || !valid || !vp || kp != key;
-    const bool tail = lane == 63 || !valid || !vn || kn != key;
-    int hv = head ? lane : 0;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        int x = __shfl_up(hv, d, 64);
-        if (lane >= d && x > hv) hv = x;
-    }
-    int tv = tail ? lane : 63;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        int x = __shfl_down(tv, d, 64);
-        if (lane + d < 64 && x < tv) tv = x;
-    }
-    h = hv;
-    t = tv;
+    const uint64_t live = __ballot(valid);
+    const bool follows = lane != 0 && valid && ((live >> (lane - 1)) & 1ull) && kp == key;
+    const uint64_t heads = __ballot(!follows);  // lane 0 always
+    const uint64_t later = heads & ~((2ull << lane) - 1ull);
+    h = 63 - __clzll((long long)(heads & ((2ull << lane) - 1ull)));
+    t = later ? __builtin_ctzll(later) - 1 : 63;
 }
 
 __device__ inline uint32_t lanes_before(uint64_t m) {
