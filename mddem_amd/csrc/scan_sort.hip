@@ -120,9 +120,10 @@ __global__ void __launch_bounds__(kScanThreads) k_scan_apply(const uint32_t* __r
 
 // The same in one launch, for up to kDirectScan elements: a block scans
 // kDirectTile of them, four per thread, and gets the sum of those before its
-// tile by adding them up itself (at most 512 KB, from L2): 6.4 us for the
-// 24,400 cells of 256,000 LJ atoms and 7.1 us for 42,900 (one workgroup tile
-// after tile: 9.2 and 16.7), 3.4 us for 1,300. Beyond, two launches cost less
+// tile by adding them up itself (at most 512 KB, from L2): 4.7 us for the
+// 24,400 cells of 256,000 LJ atoms and 5.3 us for 42,900 (one workgroup tile
+// after tile: 9.2 and 16.7; word by word: 6.5 and 7.1), 3.0 us for 1,300.
+// Beyond, two launches cost less
 // than the sums.
 constexpr int kDirectThreads = 1024;
 constexpr int kDirectTile = kDirectThreads * 4;
@@ -144,9 +145,22 @@ __global__ void __launch_bounds__(kDirectThreads) k_scan_direct(const uint32_t* 
         const uint4 q = in4[j * kDirectThreads + tid];
         before += (q.x + q.y) + (q.z + q.w);
     }
-    uint32_t v[4];
-#pragma unroll
-    for (int k = 0; k < 4; k++) v[k] = i0 + k < n ? in[i0 + k] : 0u;
+    // (four words at a time but for the end of the array)
+    const bool whole = i0 + 4 <= n;
+    uint32_t v[4] = {0u, 0u, 0u, 0u}, ad[4] = {0u, 0u, 0u, 0u};
+    auto load4 = [&](const uint32_t* p, uint32_t* x) {
+        if (whole) {
+            const uint4 q = *reinterpret_cast<const uint4*>(p + i0);
+            x[0] = q.x;
+            x[1] = q.y;
+            x[2] = q.z;
+            x[3] = q.w;
+        } else {
+            for (int k = 0; k < 4; k++) x[k] = i0 + k < n ? p[i0 + k] : 0u;
+        }
+    };
+    load4(in, v);
+    if (out2) load4(add, ad);
     const uint32_t s = (v[0] + v[1]) + (v[2] + v[3]);
     const uint32_t inc = wave_incl_scan(s);
 #pragma unroll
@@ -162,13 +176,24 @@ __global__ void __launch_bounds__(kDirectThreads) k_scan_direct(const uint32_t* 
         run += pre[k] + (k < w ? wsum[k] : 0u);
         end += pre[k] + wsum[k];
     }
+    uint32_t r[4];
 #pragma unroll
     for (int k = 0; k < 4; k++) {
-        if (i0 + k < n) {
-            out[i0 + k] = run;
-            if (out2) out2[i0 + k] = run + add[i0 + k];
-        }
+        r[k] = run;
         run += v[k];
+    }
+    if (whole) {
+        *reinterpret_cast<uint4*>(out + i0) = make_uint4(r[0], r[1], r[2], r[3]);
+        if (out2)
+            *reinterpret_cast<uint4*>(out2 + i0) =
+                make_uint4(r[0] + ad[0], r[1] + ad[1], r[2] + ad[2], r[3] + ad[3]);
+    } else {
+        for (int k = 0; k < 4; k++) {
+            if (i0 + k < n) {
+                out[i0 + k] = r[k];
+                if (out2) out2[i0 + k] = r[k] + ad[k];
+            }
+        }
     }
     if (blockIdx.x == gridDim.x - 1 && tid == 0) {
         out[n] = end;
