@@ -1763,11 +1763,19 @@ __global__ void __launch_bounds__(kExtBlock, 3) k_contact_ext(ForceArgs a, S s) 
     const int64_t i = gt >> LG;
     const int t = int(gt & (G - 1));
     if (i >= a.n) return;
-    if (gated(a)) return;
-    begin_step(a, s);
-    const double PI = 3.141592653589793;
+    // the loads that depend on no other together with the gate, as in
+    // row_head: 63.1 -> 62.3 us per step of the bed above
+    const int stop = a.st->abort_step;
     const double4 pi = a.pos[i];
     const double4 vi = a.vel[i];
+    const uint32_t first =
+        a.use_pairs && t < a.maxnb ? a.nbr[row_addr(i, t, a.npad, a.rl)] : 0u;
+    const int listed = a.use_pairs ? int(a.nnb[i]) : 0;
+    __asm__ volatile("" ::"v"(stop), "v"(pi.x), "v"(pi.w), "v"(vi.x), "v"(vi.w), "v"(first),
+                     "v"(listed));
+    if (a.step >= 0 && stop <= a.step) return;
+    begin_step(a, s);
+    const double PI = 3.141592653589793;
     R fx = R(0), fy = R(0), fz = R(0), tx = R(0), ty = R(0), tz = R(0);
     double vw[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};  // contact virial (owned pairs)
     const uint32_t ti = a.type[i];
@@ -1775,7 +1783,7 @@ __global__ void __launch_bounds__(kExtBlock, 3) k_contact_ext(ForceArgs a, S s) 
     if (a.use_pairs) {
         const double4 wi = a.omega[i];
         const uint32_t tagi = a.tag[i];
-        int cnt = int(a.nnb[i]);
+        int cnt = listed;
         if (cnt > a.maxnb) cnt = a.maxnb;
         const uint64_t mask_in = a.cmask[i];
         uint64_t mask_out = 0ull;
@@ -1784,7 +1792,7 @@ __global__ void __launch_bounds__(kExtBlock, 3) k_contact_ext(ForceArgs a, S s) 
         const int64_t cs = a.hist_cs;
         for (int k = t; k < cnt; k += G) {
             const int64_t slot = row_addr(i, k, a.npad, a.rl);
-            const uint32_t e = a.nbr[slot];
+            const uint32_t e = k == t ? first : a.nbr[slot];
             const uint32_t j = entry_idx(e);
             const bool rev = entry_rev(e);
             const double4 pj = a.pos[j];
