@@ -123,8 +123,7 @@ __global__ void __launch_bounds__(kScanThreads) k_scan_apply(const uint32_t* __r
 // tile by adding them up itself (at most 512 KB, from L2): 4.7 us for the
 // 24,400 cells of 256,000 LJ atoms and 5.3 us for 42,900 (one workgroup tile
 // after tile: 9.2 and 16.7; word by word: 6.5 and 7.1), 3.0 us for 1,300.
-// Beyond, two launches cost less
-// than the sums.
+// Beyond, two launches cost less than the sums.
 constexpr int kDirectThreads = 1024;
 constexpr int kDirectTile = kDirectThreads * 4;
 constexpr int64_t kDirectScan = int64_t(1) << 17;

@@ -101,7 +101,7 @@ def test_every_row_layout_is_filled_alike(name, lanes):
 
 
 @pytest.mark.parametrize("name", ["lj_10", "wide_bins", "faces_90", "faces_84", "poly"])
-def test_pairs_are_the_checkers(name):
+def test_pairs_are_the_oracles(name):
     w = _case(name)
     o = oracle_from_workload(w)
     _oracle_rebuild(o)

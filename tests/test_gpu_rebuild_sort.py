@@ -2,7 +2,7 @@
 around the wavefront, the workgroup and the 1,024 particles that share an image
 total; cell counts around one scan tile (4,096) and around the largest grid
 scanned in one launch (131,072); many particles in one cell. Particle order,
-pairs and image shifts must be the checker's."""
+pairs and image shifts must be the oracle's."""
 import sys
 
 import numpy as np
@@ -55,7 +55,7 @@ CASES = {
 
 
 @pytest.mark.parametrize("name", list(CASES))
-def test_sort_and_images_are_the_checkers(name):
+def test_sort_and_images_are_the_oracles(name):
     n, bins, pile = CASES[name]
     w = _random(n, bins, seed=100 + n, pile=pile)
     o = oracle_from_workload(w)

@@ -1,6 +1,6 @@
 """The pair passes read a row's first entries before they know its length:
 rows shorter than that, empty ones, the last particles of a launch and a list
-whose rows hold fewer entries than are read ahead. Forces against the checker;
+whose rows hold fewer entries than are read ahead. Forces against the oracle;
 the layouts of the one row list against each other."""
 import sys
 
