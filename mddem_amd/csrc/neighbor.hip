@@ -984,8 +984,11 @@ __global__ void __launch_bounds__(256) k_build_rows(CellArgs a, int wpc_log2) {
                 }
                 mrev = lo;
                 // (counted whether or not it fitted: a count above maxnb asks
-                // for rows of that length)
-                if (within<UNIFORM>(cc, 0.0, mx.w, mx.w)) {
+                // for rows of that length; the test is the one that put it
+                // there, which a position that is not finite does not pass)
+                const double ox = mx.x - mx.x, oy = mx.y - mx.y, oz = mx.z - mx.z;
+                const double own = fma(ox, ox, fma(oy, oy, oz * oz));
+                if (within<UNIFORM>(cc, own, mx.w, mx.w)) {
                     self = lo;
                     mcnt--;
                 }
