@@ -995,6 +995,7 @@ int mdd_clear_walls(mdd_ctx* ctx) {
         c.walls.count = 0;
         c.walls_moving = false;
         c.wdyn.release();
+        c.wdyn2.release();
         c.walls_dev.release();
     });
 }

@@ -574,7 +574,7 @@ void swap_state(Ctx& c) {
 
 void swap_step_buffers(Ctx& c) {
     swap_state(c);
-    if (c.wdyn2.p) c.wdyn.swap(c.wdyn2);
+    if (c.walls.count > 0) c.wdyn.swap(c.wdyn2);  // as the pass had them (step_args)
 }
 
 // scheduled post kernel of a step; its thermostat half uses slot step & 1
