@@ -184,11 +184,14 @@ void run_steps(Ctx& c, int64_t nsteps) {
         c.post_pending = false;
     }
     // pre_done: the step whose first half the last force pass did already;
+    // paired: it did, and the buffers are as it left them (IntArgs::paired);
     // fused: the passes of the running chunk that integrate, newest last
     int pre_done = -1;
+    bool paired = false;
     std::vector<int> fused;
     auto first_half = [&](int s, bool check) {
         if (s == pre_done) return;
+        paired = false;
         if (c.post_pending) {
             mdd::launch_post_pre(c, s, check);
             c.post_pending = false;
@@ -212,13 +215,15 @@ void run_steps(Ctx& c, int64_t nsteps) {
     // step s + 1 in the same launch unless the run ends or the list is due
     auto force_pass = [&](int s) {
         if (s < end && !count_due(int64_t(s) + 1) && mdd::step_fusable(c, s)) {
-            mdd::launch_pair_forces(c, s, false, true);
+            mdd::launch_pair_forces(c, s, false, true, paired);
             mdd::swap_step_buffers(c);
             fused.push_back(s);
             pre_done = s + 1;
+            paired = true;
             c.post_pending = false;
         } else {
             pre_done = -1;
+            paired = false;
             mdd::launch_pair_forces(c, s, false);
             second_half(s);
         }
@@ -243,6 +248,7 @@ void run_steps(Ctx& c, int64_t nsteps) {
         if (ab != c.last_resume) c.repeats = 0;
         c.last_resume = ab;
         mdd::rebuild_async(c, ab, retry);
+        paired = false;
         if (!retry) c.last_rebuild = ab;
         force_pass(ab);
         if (!retry) {
@@ -262,9 +268,13 @@ void run_steps(Ctx& c, int64_t nsteps) {
     auto check_status = [&]() {
         sync_status(c);
         harvest_profile(c);
-        // passes at or past the abort step did not run: their buffers go back
+        // passes at or past the abort step did not run, or the overlap limit
+        // stopped them: their buffers go back
         const int ab = c.status_host->abort_step;
-        for (; !fused.empty() && fused.back() >= ab; fused.pop_back()) mdd::swap_step_buffers(c);
+        for (; !fused.empty() && fused.back() >= ab; fused.pop_back()) {
+            mdd::swap_step_buffers(c);
+            paired = false;
+        }
         fused.clear();
         check_device_error(c);
         return ab;
@@ -278,6 +288,7 @@ void run_steps(Ctx& c, int64_t nsteps) {
                 // FullRebuild step: integrate, rebuild, force, integrate
                 first_half(int(s), false);
                 mdd::rebuild_async(c, int(s), false);
+                paired = false;
                 c.last_rebuild = s;
                 force_pass(int(s));
                 c.step = s;

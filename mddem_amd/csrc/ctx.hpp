@@ -417,9 +417,9 @@ struct Ctx {
     DBuf<float> f32, t32;   // 3*npad SoA force / torque (mixed mode)
     DBuf<double4> build_pos;
     // the other side of a force pass that integrates (allocated by the first
-    // one): swapped with pos / vel / omega at each such pass; third: pos, vel
-    // and omega are now the buffers these members started with
-    DBuf<double4> pos3, vel3, omega3;
+    // one): swapped with pos / vel / omega / quat at each such pass; third:
+    // those are now the buffers these members started with
+    DBuf<double4> pos3, vel3, omega3, quat3;
     bool third = false;
     bool sorted_third = false;  // third at the last sort (its source)
     // alternates for the rebuild permutation
@@ -605,8 +605,10 @@ void launch_sort_check(Ctx& c, int step);
 void release_graphs(Ctx& c);
 bool rebuild_grow(Ctx& c, const Status& s);
 // forces.hip
-// integrate: the pass goes on to the next step's first half (step_fusable)
-void launch_pair_forces(Ctx& c, int step, bool energy, bool integrate = false);
+// integrate: the pass goes on to the next step's first half (step_fusable);
+// paired: IntArgs::paired
+void launch_pair_forces(Ctx& c, int step, bool energy, bool integrate = false,
+                        bool paired = false);
 void launch_walls_gravity(Ctx& c, bool walls, bool gravity);
 // standalone wall_move / wall_zero_force_accumulators
 void launch_wall_systems(Ctx& c, bool move, bool zero);

@@ -2307,7 +2307,7 @@ void upload_materials(Ctx& c) {
 }
 
 // one pair-force pass (Force phase). step < 0: ungated standalone call.
-void launch_pair_forces(Ctx& c, int step, bool energy, bool integrate) {
+void launch_pair_forces(Ctx& c, int step, bool energy, bool integrate, bool paired) {
     ForceArgs a = make_args(c, step);
     const bool mixed = c.precision == 1;
     if (step < 0) {
@@ -2377,7 +2377,7 @@ void launch_pair_forces(Ctx& c, int step, bool energy, bool integrate) {
         } else {
             if (mixed && c.xq_usable()) lj_fixed_setup(c, a);
             if (integrate) {
-                const StepArgs s = step_args(c, step);
+                const StepArgs s = step_args(c, step, paired);
                 if (mixed)
                     launch_lj<float, false>(c, a, s, k0, k1);
                 else
@@ -2406,7 +2406,7 @@ void launch_pair_forces(Ctx& c, int step, bool energy, bool integrate) {
             else
                 launch_hertz<double, true>(c, a, NoStep{}, k0, k1);
         } else if (integrate) {
-            const StepArgs s = step_args(c, step);
+            const StepArgs s = step_args(c, step, paired);
             if (mixed)
                 launch_dem<float>(c, a, s, split, k0, k1);
             else

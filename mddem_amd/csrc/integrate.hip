@@ -92,7 +92,7 @@ __device__ inline void rotate_initial(const IntArgs& a, int64_t i, double tx, do
     w.z += 0.5 * dt * tz * ii;
     // a zero torque leaves the spin as it is: no store
     if (tx != 0.0 || ty != 0.0 || tz != 0.0) a.omega[i] = w;
-    rotate_quat(a, i, w);
+    rotate_quat(a, i, w, a.quat, false);
 }
 
 // final_rotation body (rotational.rs:87-100)
@@ -275,7 +275,7 @@ __global__ void __launch_bounds__(kThreads) k_post_pre(IntArgs a) {
             w.z += 0.5 * dt * tz * ii;
             // a zero torque leaves the spin as it is: no store
             if (tx != 0.0 || ty != 0.0 || tz != 0.0) a.omega[i] = w;
-            rotate_quat(a, i, w);
+            rotate_quat(a, i, w, a.quat, false);
         }
     }
     if (a.check) rebuild_check(a, i, p, b);
@@ -539,18 +539,21 @@ bool step_fusable(const Ctx& c, int step) {
     return !(c.model == 1 && c.nsys == 0 && c.virial_every > 0 && step % c.virial_every == 0);
 }
 
-StepArgs step_args(Ctx& c, int step) {
+StepArgs step_args(Ctx& c, int step, bool paired) {
     StepArgs s{};
     s.in = integrate_args(c, step + 1, true);
     s.in.vv = c.vv_on;
     s.in.rot = c.rot_on && c.model == 1;
     c.pos3.resize(size_t(c.npad));
     c.vel3.resize(size_t(c.npad));
+    s.in.paired = paired ? 1 : 0;
     s.pos = c.pos3.p;
     s.vel = c.vel3.p;
     if (c.model == 1) {
         c.omega3.resize(size_t(c.npad));
+        c.quat3.resize(size_t(c.npad));
         s.omega = c.omega3.p;
+        s.quat = c.quat3.p;
     }
     if (s.in.xq) {
         c.xq2.resize(size_t(c.npad));
@@ -567,7 +570,10 @@ StepArgs step_args(Ctx& c, int step) {
 void swap_state(Ctx& c) {
     c.pos.swap(c.pos3);
     c.vel.swap(c.vel3);
-    if (c.model == 1) c.omega.swap(c.omega3);
+    if (c.model == 1) {
+        c.omega.swap(c.omega3);
+        c.quat.swap(c.quat3);
+    }
     if (c.xq2.p) c.xq.swap(c.xq2);
     c.third = !c.third;
 }

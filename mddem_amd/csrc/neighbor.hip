@@ -132,7 +132,7 @@ struct PermArgs {
     int64_t n, npad;
     const uint32_t* order;
     const double4 *pos, *vel, *omega, *quat;
-    const double4 *pos3, *vel3, *omega3;  // their sources when st->third
+    const double4 *pos3, *vel3, *omega3, *quat3;  // their sources when st->third
     const Status* st;
     double4 *pos2, *vel2, *omega2, *quat2, *build_pos;
     const uint32_t *tag, *type, *key;
@@ -209,6 +209,7 @@ __global__ void __launch_bounds__(256) k_permute(PermArgs a) {
             a.pos = a.pos3;
             a.vel = a.vel3;
             a.omega = a.omega3;
+            a.quat = a.quat3;
         }
         uint32_t o;
         if (PLACED) {
@@ -1601,6 +1602,7 @@ void permute_all(Ctx& c, bool placed, int64_t n) {
     a.pos3 = c.pos3.p;
     a.vel3 = c.vel3.p;
     a.omega3 = c.omega3.p;
+    a.quat3 = c.quat3.p;
     a.st = c.status.p;
     a.quat = c.quat.p;
     a.pos2 = c.pos2.p;

@@ -23,6 +23,9 @@ struct IntArgs {
     int rot;         // apply rotation half-steps
     int vv;          // apply Verlet translational half-steps
     int check;       // evaluate the rebuild decision
+    int paired;      // StepArgs: the first half of the step before was such a pass too, and
+                     // nothing has written an orientation since, so spheres that it did not
+                     // turn have the same one in both buffers
     double thr2;     // ((skin_fraction - 1) * min_skin)^2
     BoxP box;
     int box_exit;
@@ -134,25 +137,29 @@ __device__ inline void rebuild_check_fixed(const IntArgs& a, int64_t i, const do
 }
 
 // orientation update of initial_rotation with the kicked omega w
-// (rotational.rs:70-83)
-__device__ inline void rotate_quat(const IntArgs& a, int64_t i, const double4& w) {
+// (rotational.rs:70-83) into quat[i]; `keep`: the orientation goes there also
+// where the spin is too slow to turn it
+__device__ inline void rotate_quat(const IntArgs& a, int64_t i, const double4& w, double4* quat,
+                                   bool keep) {
     const double dt = a.dt;
     const double omega_mag = sqrt(w.x * w.x + w.y * w.y + w.z * w.z);
     const double angle = omega_mag * dt;
-    if (angle > 1e-14) {
+    const bool turns = angle > 1e-14;
+    if (!turns && !keep) return;
+    const double4 b = a.quat[i];
+    double4 q = b;
+    if (turns) {
         const double inv = 1.0 / omega_mag;
         const double ax = w.x * inv, ay = w.y * inv, az = w.z * inv;
         const double half = angle * 0.5;
         const double s = sin(half);
         const double a0 = cos(half), a1 = ax * s, a2 = ay * s, a3 = az * s;
-        const double4 b = a.quat[i];
-        double4 q;
         q.x = a0 * b.x - a1 * b.y - a2 * b.z - a3 * b.w;
         q.y = a0 * b.y + a1 * b.x + a2 * b.w - a3 * b.z;
         q.z = a0 * b.z - a1 * b.w + a2 * b.x + a3 * b.y;
         q.w = a0 * b.w + a1 * b.z - a2 * b.y + a3 * b.x;
-        a.quat[i] = q;
     }
+    quat[i] = q;
 }
 
 __device__ inline void kick_drift(const IntArgs& a, double4& v, double4& p, double fx, double fy,
@@ -169,11 +176,14 @@ __device__ inline void kick_drift(const IntArgs& a, double4& v, double4& p, doub
 
 // Where a force pass that integrates writes the new state: buffers other
 // than the ones it reads (neighbors' positions, velocities and spins are
-// read while others already advance), exchanged by the host after the launch.
+// read while others already advance, and a pass that the overlap limit stops
+// midway leaves the old state whole), exchanged by the host after the launch.
+// (the orientations' own buffer: 0.1 us of 12.5 at 200,000 gas spheres, 0.3 of
+// 19.1 on a bed of 62,500, against turning them in place)
 // wdyn is the coming step's wall state.
 struct StepArgs {
     IntArgs in;  // of the coming step
-    double4 *pos, *vel, *omega;
+    double4 *pos, *vel, *omega, *quat;
     WallsDyn* wdyn;
 };
 struct NoStep {};
@@ -200,6 +210,7 @@ __device__ inline void step_begin(const StepArgs& s, const WallsDyn* now) {
 struct StepIn {
     double4 v, w, b;
     int4 bq;
+    bool stale;  // the other buffer may hold another orientation than this one
 };
 
 __device__ inline StepIn step_load(const StepArgs& s, int64_t i) {
@@ -207,6 +218,8 @@ __device__ inline StepIn step_load(const StepArgs& s, int64_t i) {
     StepIn x;
     x.v = a.vel[i];
     x.w = s.omega ? a.omega[i] : make_double4(0.0, 0.0, 0.0, 0.0);
+    // (w is the spin that the last first half turned the orientation with)
+    x.stale = !a.paired || x.w.x != 0.0 || x.w.y != 0.0 || x.w.z != 0.0;
     x.b = make_double4(0.0, 0.0, 0.0, 0.0);
     x.bq = make_int4(0, 0, 0, 0);
     if (a.check) {
@@ -246,7 +259,9 @@ __device__ inline void step_advance(const StepArgs& s, int64_t i, double4 p, con
                 w.y += 0.5 * dt * ty * ii;
                 w.z += 0.5 * dt * tz * ii;
             }
-            rotate_quat(a, i, w);
+            rotate_quat(a, i, w, s.quat, x.stale);
+        } else if (x.stale) {
+            s.quat[i] = a.quat[i];
         }
         s.omega[i] = w;
     }
@@ -263,6 +278,6 @@ __device__ inline void step_advance(const StepArgs& s, int64_t i, double4 p, con
 // third buffers; swap_step_buffers exchanges them after the launch, or back
 // for a pass that the device did not run)
 IntArgs integrate_args(Ctx& c, int step, bool check);
-StepArgs step_args(Ctx& c, int step);
+StepArgs step_args(Ctx& c, int step, bool paired);
 
 }  // namespace mdd
