@@ -141,6 +141,8 @@ void download(Ctx& c, const Column* cols, int ncols, int64_t n) {
         pack(c, pieces[size_t(q)], s + size_t(q % slots) * kSlot);
         MDD_HIP(hipEventRecord(c.stage_ev[size_t(q % slots)], c.stream));
     };
+    std::vector<std::thread> threads;
+    threads.reserve(size_t(copiers));
     for (int q = 0; q < slots; q++) issue(q);
     std::mutex mu;  // one thread launches and records at a time
     std::exception_ptr failed;
@@ -164,15 +166,17 @@ void download(Ctx& c, const Column* cols, int ncols, int64_t n) {
             stop.store(true);
         }
     };
-    std::vector<std::thread> threads;
-    try {
-        for (int t = 1; t < copiers; t++) threads.emplace_back(copier, t);
-    } catch (...) {  // no more threads to be had
-        std::lock_guard<std::mutex> lk(mu);
-        failed = std::current_exception();
-        stop.store(true);
+    // a copier that gets no thread of its own has its turn on this one
+    int own = copiers;
+    for (int t = 1; t < own; t++) {
+        try {
+            threads.emplace_back(copier, t);
+        } catch (...) {  // no more threads to be had
+            own = t;
+        }
     }
-    if (!stop.load()) copier(0);
+    copier(0);
+    for (int t = own; t < copiers; t++) copier(t);
     for (auto& th : threads) th.join();
     if (failed) {
         (void)hipStreamSynchronize(c.stream);
