@@ -31,7 +31,7 @@ from mddem_amd import workloads as W
 
 # device bytes per particle (state, forces, alternates, neighbor rows,
 # shear history, bins) used to admit jobs; measured allocations stay below
-FOOTPRINT_PER_PARTICLE = {"dem": 3200, "lj": 1400}
+FOOTPRINT_PER_PARTICLE = {"dem": 3200, "lj": 1500}
 FOOTPRINT_FIXED = 64 << 20
 
 
