@@ -556,7 +556,9 @@ struct Ctx {
     int64_t last_resume = -1;  // step of the last rebuild inside a run and
     int repeats = 0;           // how many times in a row it was that step
 
-    // ---- pinned staging memory of downloads, one event per slot
+    // ---- pinned staging memory of downloads (from the second on), one event
+    // per slot
+    bool downloaded = false;
     char* stage = nullptr;
     size_t stage_bytes = 0;
     std::vector<hipEvent_t> stage_ev;

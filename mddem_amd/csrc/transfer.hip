@@ -10,10 +10,17 @@
 // slower side (a few GB/s on one thread), so large downloads use several
 // threads, each on its own pieces. Single-precision forces cross the bus as
 // they are and become doubles on their way to the caller's array.
+//
+// A context's first download, unless it is large, goes without the pinned
+// memory, whose allocation and release take 0.3 to 0.7 ms: a job that runs and
+// takes its state once would not see them again (the state of 50,000 spheres:
+// 0.70 ms without, 1.0 and 0.4 at the end with it; from 8 MiB on, the pinned
+// pieces are faster even so, 200,000 spheres 1.8 ms instead of 3.4).
 #include <algorithm>
 #include <atomic>
 #include <cstring>
 #include <exception>
+#include <memory>
 #include <mutex>
 #include <thread>
 
@@ -83,16 +90,52 @@ void place(const Piece& p, const void* from) {
     std::memcpy(to, from, size_t(p.count) * row_bytes(k));
 }
 
-// `raw`: a soa32 column's device array as it is
+// `raw`: the column's device array as it is
 void unpack(const Column& col, const void* raw, int64_t npad, int64_t n) {
+    const double* q = static_cast<const double*>(raw);
+    const int32_t* q32 = static_cast<const int32_t*>(raw);
     const float* f = static_cast<const float*>(raw);
     double* out = static_cast<double*>(col.host);
-    for (int64_t i = 0; i < n; i++)
-        for (int d = 0; d < 3; d++) out[3 * i + d] = double(f[d * npad + i]);
+    int32_t* out32 = static_cast<int32_t*>(col.host);
+    switch (col.kind) {
+        case ColumnKind::u32:
+        case ColumnKind::f64:
+        case ColumnKind::xyzw: std::memcpy(out, raw, size_t(n) * row_bytes(col.kind)); break;
+        case ColumnKind::w:
+            for (int64_t i = 0; i < n; i++) out[i] = q[4 * i + 3];
+            break;
+        case ColumnKind::xyz:
+            for (int64_t i = 0; i < n; i++)
+                for (int d = 0; d < 3; d++) out[3 * i + d] = q[4 * i + d];
+            break;
+        case ColumnKind::ixyz:
+            for (int64_t i = 0; i < n; i++)
+                for (int d = 0; d < 3; d++) out32[3 * i + d] = q32[4 * i + d];
+            break;
+        case ColumnKind::soa32:
+            for (int64_t i = 0; i < n; i++)
+                for (int d = 0; d < 3; d++) out[3 * i + d] = double(f[d * npad + i]);
+            break;
+        case ColumnKind::soa64:
+            for (int64_t i = 0; i < n; i++)
+                for (int d = 0; d < 3; d++) out[3 * i + d] = q[d * npad + i];
+            break;
+    }
+}
+size_t raw_bytes(ColumnKind k, int64_t npad, int64_t n) {
+    switch (k) {
+        case ColumnKind::u32: return 4 * size_t(n);
+        case ColumnKind::f64: return 8 * size_t(n);
+        case ColumnKind::ixyz: return 16 * size_t(n);
+        case ColumnKind::soa32: return 12 * size_t(npad);
+        case ColumnKind::soa64: return 24 * size_t(npad);
+        default: return 32 * size_t(n);
+    }
 }
 
 constexpr size_t kSlot = size_t(1) << 19;  // bytes of one piece
 constexpr int kMaxCopiers = 8;             // host threads of one download
+constexpr size_t kPlain = size_t(8) << 20; // a first download below goes without them
 
 // pinned staging memory of at least `bytes`, kept with the context
 char* staging(Ctx& c, size_t bytes) {
@@ -120,6 +163,18 @@ void download(Ctx& c, const Column* cols, int ncols, int64_t n) {
     size_t total = 0;
     for (int k = 0; k < ncols; k++) total += row_bytes(cols[k].kind) * size_t(n);
     if (total == 0) return;
+    if (!c.downloaded && total < kPlain) {
+        size_t most = 0;
+        for (int k = 0; k < ncols; k++) most = std::max(most, raw_bytes(cols[k].kind, c.npad, n));
+        const std::unique_ptr<char[]> raw(new char[most]);
+        for (int k = 0; k < ncols; k++) {
+            d2h(c, raw.get(), cols[k].dev, raw_bytes(cols[k].kind, c.npad, n));
+            unpack(cols[k], raw.get(), c.npad, n);
+        }
+        c.downloaded = true;
+        return;
+    }
+    c.downloaded = true;
     // up to 2 MiB (tens of thousands of particles): every column packed, one
     // wait, one thread. Single-precision forces are copied as they are and
     // picked here: at 20,000 atoms a force download takes 26 us, 32 with them
@@ -127,7 +182,7 @@ void download(Ctx& c, const Column* cols, int ncols, int64_t n) {
     if (total <= (size_t(2) << 20)) {
         auto plain = [](const Column& col) { return col.kind == ColumnKind::soa32; };
         auto bytes = [&](const Column& col) {
-            return plain(col) ? 12 * size_t(c.npad) : row_bytes(col.kind) * size_t(n);
+            return plain(col) ? raw_bytes(col.kind, c.npad, n) : row_bytes(col.kind) * size_t(n);
         };
         size_t all = 0, at = 0;
         for (int k = 0; k < ncols; k++) all += bytes(cols[k]);
