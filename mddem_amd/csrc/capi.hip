@@ -179,6 +179,7 @@ void run_steps(Ctx& c, int64_t nsteps) {
     // half step and the next step's first: the final half is deferred and
     // issued together with the next first half (one pass over the state).
     const bool defer = !c.nh_on;
+    const bool one_launch = mdd::one_launch_pays(c, end);
     if (c.post_pending) {
         mdd::launch_post(c, int(c.step));
         c.post_pending = false;
@@ -214,7 +215,7 @@ void run_steps(Ctx& c, int64_t nsteps) {
     // the force pass of step s and what follows it: on to the first half of
     // step s + 1 in the same launch unless the run ends or the list is due
     auto force_pass = [&](int s) {
-        if (s < end && !count_due(int64_t(s) + 1) && mdd::step_fusable(c, s)) {
+        if (s < end && one_launch && !count_due(int64_t(s) + 1) && mdd::step_fusable(c, s)) {
             mdd::launch_pair_forces(c, s, false, true, paired);
             mdd::swap_step_buffers(c);
             fused.push_back(s);

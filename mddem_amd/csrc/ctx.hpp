@@ -273,12 +273,13 @@ template <class T>
 struct DBuf {
     T* p = nullptr;
     size_t n = 0;
+    bool part = false;  // of another buffer, which frees it
     DBuf() = default;
     DBuf(const DBuf&) = delete;
     DBuf& operator=(const DBuf&) = delete;
     ~DBuf() { release(); }
     void release() {
-        if (p) {
+        if (p && !part) {
             // while launches are being recorded, a buffer they name stays
             // allocated until they have been issued
             if (deferred_frees())
@@ -288,6 +289,7 @@ struct DBuf {
         }
         p = nullptr;
         n = 0;
+        part = false;
     }
     void resize(size_t count) {
         if (count <= n && p) return;
@@ -299,6 +301,13 @@ struct DBuf {
     void swap(DBuf& o) {
         std::swap(p, o.p);
         std::swap(n, o.n);
+        std::swap(part, o.part);
+    }
+    void set_part(T* at, size_t count) {
+        release();
+        p = at;
+        n = count;
+        part = true;
     }
 };
 
@@ -420,8 +429,9 @@ struct Ctx {
     DBuf<double4> build_pos;
     // the other side of a force pass that integrates (allocated by the first
     // one): swapped with pos / vel / omega / quat at each such pass; third:
-    // those are now the buffers these members started with
-    DBuf<double4> pos3, vel3, omega3, quat3;
+    // those are now the buffers these members started with. One allocation
+    // (third_mem): a context pays some 0.25 ms for each of several.
+    DBuf<double4> third_mem, pos3, vel3, omega3, quat3;
     bool third = false;
     bool sorted_third = false;  // third at the last sort (its source)
     // alternates for the rebuild permutation
@@ -633,6 +643,8 @@ inline void set_contact_path(Ctx& c, bool on) {
 }
 // integrate.hip
 bool step_fusable(const Ctx& c, int step);
+// whether a run up to step `end` of a context's life repays the third buffers
+bool one_launch_pays(const Ctx& c, int64_t end);
 void swap_step_buffers(Ctx& c);
 void swap_state(Ctx& c);
 void launch_pre(Ctx& c, int step, bool check_rebuild);
