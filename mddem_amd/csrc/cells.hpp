@@ -14,12 +14,7 @@ __device__ inline uint32_t xcd_block(uint32_t b, uint32_t nb) {
     return (x < r ? x * (q + 1u) : r * (q + 1u) + (x - r) * q) + i;
 }
 
-// lanes above / below lane `rel` of a 64-lane chunk
-__device__ inline uint64_t lanes_above(int rel) {
-    if (rel < 0) return ~0ull;
-    if (rel >= 63) return 0ull;
-    return ~0ull << (rel + 1);
-}
+// lanes below lane `rel` of a 64-lane chunk
 __device__ inline uint64_t lanes_below(int rel) {
     if (rel <= 0) return 0ull;
     if (rel >= 64) return ~0ull;

@@ -496,9 +496,6 @@ struct Ctx {
     // the final half step of step `step` is deferred into the next step's
     // first pass (runs without a thermostat)
     bool post_pending = false;
-    // runs without a thermostat: the force pass of a step does that step's
-    // final half and the next step's first half as well, one launch per step
-    bool step_fused = true;
     // neighbor build kernel: 0 chosen by occupancy, 1 one wavefront per cell,
     // 2 one lane per member slot (sparse grids)
     int build_mode = 0;

@@ -531,7 +531,7 @@ void launch_post_pre(Ctx& c, int step, bool check_rebuild) {
 // their own after the pair pass), no contact virial of this step (its kernel
 // stores the forces) and no cell tiles.
 bool step_fusable(const Ctx& c, int step) {
-    if (!c.step_fused || c.nh_on || !c.vv_on || c.walls_moving || c.list_tile ||
+    if (c.nh_on || !c.vv_on || c.walls_moving || c.list_tile ||
         c.list_injected || !c.list_valid)
         return false;
     for (int k = 0; k < c.walls.count; k++)

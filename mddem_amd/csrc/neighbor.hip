@@ -249,7 +249,8 @@ __global__ void __launch_bounds__(256) k_permute(PermArgs a) {
                 for (int d = 0; d < 3; d++) a.t64b[d * a.npad + k] = a.t64[d * a.npad + o];
             if (a.t32)
                 for (int d = 0; d < 3; d++) a.t32b[d * a.npad + k] = a.t32[d * a.npad + o];
-        }        BoxP box = a.box;
+        }
+        BoxP box = a.box;
         double gc = a.gc;
         if (a.sysp) {
             const SysP& S = a.sysp[a.psys[k]];
@@ -2146,9 +2147,6 @@ void release_graphs(Ctx& c) {
     c.graphs.clear();
 }
 
-// One rebuild. A first attempt (not a retry) is recorded and issued as a
-// graph: its launches (10 for LJ) reach the device at once instead of one host
-// launch at a time.
 void launch_sort_check(Ctx& c, int step) {
     if (c.n < 2) return;
     launch(c, k_sort_check, blocks_for(c.n, 256), 256, c.n, static_cast<const double4*>(c.pos.p),
@@ -2156,6 +2154,9 @@ void launch_sort_check(Ctx& c, int step) {
     MDD_HIP(hipGetLastError());
 }
 
+// One rebuild. A first attempt (not a retry) is recorded and issued as a
+// graph: its launches (10 for LJ, after the one that begins it) reach the device
+// at once instead of one host launch at a time.
 void rebuild_async(Ctx& c, int step, bool retry) {
     const bool timed = c.prof_every > 0 && c.rb_pending < int64_t(c.rb_ev.size() / 3);
     if (timed) {
