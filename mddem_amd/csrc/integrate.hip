@@ -530,7 +530,22 @@ void launch_post_pre(Ctx& c, int step, bool check_rebuild) {
 // motion may depend on the whole pass' force sum), no region walls (a pass of
 // their own after the pair pass), no contact virial of this step (its kernel
 // stores the forces) and no cell tiles.
+// With several lanes a particle, one of them integrates while the others wait,
+// and a pass of its own has every lane at work: at eight lanes up to 50,000
+// spheres or 210,000 atoms, at four up to 200,000 spheres. In us per step, with
+// and without: eight lanes, a bed of 20,000 15.0 / 16.1, of 40,000 21.1 / 21.3,
+// of 62,500 30.1 / 28.4, of 150,000 62.8 / 56.2, LJ 108,000 31.8 / 35.5, 203,000
+// 48.0 / 51.0 (64-bit 65.8 / 66.1), 500,000 104 / 99; four lanes, a gas of
+// 100,000 11.6 / 12.5, of 300,000 26.5 / 26.0, a bed of 150,000 43.3 / 44.8, of
+// 500,000 121 / 117, one with adhesion of 140,000 50.0 / 52.7, of 500,000 173 /
+// 155; LJ at four lanes 500,000 89 / 97.
 bool step_fusable(const Ctx& c, int step) {
+    if (c.model == 1) {
+        const int lg = c.lanes_auto && !c.ext_on ? 0 : c.list_lanes;
+        if (lg >= 2 && c.n >= (lg == 3 ? 50000 : 200000)) return false;
+    } else if (c.list_lanes == 3 && c.n > 210000) {
+        return false;
+    }
     if (c.nh_on || !c.vv_on || c.walls_moving || c.list_tile ||
         c.list_injected || !c.list_valid)
         return false;
