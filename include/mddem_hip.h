@@ -318,9 +318,10 @@ int mdd_device_memory(int device, int64_t* free_bytes, int64_t* total_bytes);
 /* DEM force pass at one lane per particle (log2 lanes 0): -1 (default)
  * split by row length (particles with neighbors in the pair kernel, the
  * rest in a walls-and-gravity kernel) when fewer than half the particles
- * had neighbors at the last build the host has seen, else one kernel; 0
- * always one kernel; 1 always split. Identical forces. No reference
- * counterpart: launch-shape tuning. */
+ * had neighbors at the last build the host has seen, and the pass does not
+ * advance the particles as well (steps in one launch, runs without a
+ * thermostat), else one kernel; 0 always one kernel; 1 always split.
+ * Identical forces. No reference counterpart: launch-shape tuning. */
 int mdd_set_dem_split(mdd_ctx* ctx, int mode);
 /* DEM pair pass (single systems, rows of any lane count) in tile order:
  * on (default) the particles are visited band of bin columns by band (16

@@ -43,6 +43,25 @@ def _runs_alike(w, prec, configure):
     b.close()
 
 
+def _cloud_on_a_floor(n):
+    # spheres moving between two planes under gravity
+    w = W.dem_settling(n=n, box=(0.06, 0.06, 0.3))
+    w.vel = (W.Stream(9).uniform(3 * n).reshape(-1, 3) - 0.5) * 4.0
+    w.omega = (W.Stream(6).uniform(3 * n).reshape(-1, 3) - 0.5) * 100.0
+    return w
+
+
+@pytest.mark.parametrize("prec", [hip.MIXED, hip.FP64])
+@pytest.mark.parametrize("split", [-1, 1])
+@pytest.mark.parametrize("n", [1, 257, 3001])
+def test_split_by_row_length(n, split, prec):
+    def configure(s):
+        s.set_force_lanes(0)
+        s.set_dem_split(split)
+
+    _runs_alike(_cloud_on_a_floor(n), prec, configure)
+
+
 @pytest.mark.parametrize("prec", [hip.MIXED, hip.FP64])
 @pytest.mark.parametrize("lanes,n", [(3, 49999), (3, 50000), (2, 199999), (2, 200000)])
 def test_lanes(lanes, n, prec):
