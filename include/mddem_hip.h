@@ -353,11 +353,15 @@ int mdd_set_lj_post_fused(mdd_ctx* ctx, int on);
  * geometry in FP64. No reference counterpart: precision/speed choice of
  * the mixed path. */
 int mdd_set_lj_positions(mdd_ctx* ctx, int mode);
-/* Pair-force layout: log2 lanes per particle of the row kernels (0..3;
- * default 2), or -1 for the LJ cell-tile kernel (16-bit rows into each bin
- * cell's candidate list staged in LDS; LJ contexts only, others keep rows).
- * Changes the neighbor-row layout, so the next step rebuilds the list. No
- * reference counterpart: launch-shape tuning. */
+/* Pair-force layout: log2 lanes per particle of the row kernels (0..3), or
+ * -1 for the LJ cell-tile kernel (16-bit rows into each bin cell's candidate
+ * list staged in LDS; LJ contexts only, others keep rows). Until it is called
+ * LJ contexts run at 2 (four lanes), DEM contexts at one or two lanes by the
+ * number of spheres and the length of their rows, with the sums in the order
+ * of four lanes: the same forces, bit for bit, as at 2. A choice other than
+ * the current one (before the first: other than 2) changes the neighbor-row
+ * layout, so the next step rebuilds the list. No reference counterpart:
+ * launch-shape tuning. */
 int mdd_set_force_lanes(mdd_ctx* ctx, int log2_lanes);
 /* Neighbor-row build kernel: 0 (default) picks by grid occupancy, 1 one
  * wavefront per bin cell, 2 one lane per particle or image (for sparse grids

@@ -1620,7 +1620,9 @@ int mdd_set_force_lanes(mdd_ctx* ctx, int log2_lanes) {
     return guarded(ctx, [&](Ctx& c) {
         if (log2_lanes < -1 || log2_lanes > 3)
             throw ApiError(MDD_ERR_INVALID, "log2 lanes per particle must be -1..3");
-        // the next step rebuilds the list in the new layout
+        // the next step rebuilds the list if the lanes differ; rows that an
+        // automatic DEM context laid out for two lanes are read as they are
+        // (ForceArgs::rl) until the next rebuild
         c.tile_enabled = log2_lanes < 0;
         if (log2_lanes >= 0) {
             c.lanes = log2_lanes;

@@ -575,7 +575,8 @@ class System:
 
     def set_force_lanes(self, log2_lanes: int):
         """Row kernels at 2^log2_lanes lanes per particle (0..3), or the LJ
-        cell-tile kernel (-1)."""
+        cell-tile kernel (-1). Before the first call: LJ four lanes, DEM one
+        or two chosen by size, with the forces of four bit for bit."""
         self._c(self.L.mdd_set_force_lanes(self.h, int(log2_lanes)))
 
     def set_build_kernel(self, mode: int):
