@@ -70,3 +70,69 @@ def test_short_runs_and_a_long_one(kind):
         _same(a, b)
     a.close()
     b.close()
+
+
+def test_a_long_run_makes_the_copy():
+    # 50,000 spheres: 6.4 MB of second state after run(40), none after 40 x run(1)
+    w = W.gas_system(50000, 0.2, 0.9, 0.4, seed=3)
+    used = []
+    for calls in ((40,), (1,) * 40):
+        free = hip.device_memory(0)[0]
+        s = hip.from_workload(w, hip.MIXED, box_exit=False)
+        for k in calls:
+            s.run(k)
+        used.append(free - hip.device_memory(0)[0])
+        s.close()
+    assert used[0] - used[1] >= 4 * 32 * w.n - (2 << 20)
+
+
+def _pair(w, prec, n, configure=lambda s: None):
+    a, b = (hip.from_workload(w, prec, box_exit=False) for _ in range(2))
+    configure(a)
+    configure(b)
+    a.run(n)
+    for _ in range(n):
+        b.run(1)
+    return a, b
+
+
+@pytest.mark.parametrize("prec", [hip.MIXED, hip.FP64])
+@pytest.mark.parametrize("sign", [-1.0, 1.0])
+def test_rebuilds_that_do_not_fit(sign, prec):
+    # inward: rows outgrow their capacity; outward: the images near the faces do
+    w = W.lj_fcc(ncell=5, rho=0.3, thermostat=False)
+    L = w.hi - w.lo
+    d = w.pos - (w.lo + 0.5 * L)
+    d -= L * np.round(d / L)
+    w.vel = sign * 1.2 * d / (0.5 * L)
+    a, b = _pair(w, prec, 300)
+    assert a.thermo()["rebuilds"] == b.thermo()["rebuilds"] > 3
+    _same(a, b)
+    a.close()
+    b.close()
+
+
+@pytest.mark.parametrize("prec", [hip.MIXED, hip.FP64])
+@pytest.mark.parametrize("steps", [400, 401])
+def test_spheres_that_leave_through_fixed_faces(steps, prec):
+    w = W.gas_system(700, 0.3, 0.9, 0.4, seed=3)
+    w.vel = w.vel * 40.0
+    w.omega = (W.Stream(6).uniform(3 * w.n).reshape(-1, 3) - 0.5) * 100.0
+    w.periodic = (False, True, False)
+    a, b = _pair(w, prec, steps)
+    assert a.n == b.n and 100 < a.n < w.n - 20
+    _same(a, b)
+    a.close()
+    b.close()
+
+
+@pytest.mark.parametrize("prec", [hip.MIXED, hip.FP64])
+@pytest.mark.parametrize("every", [2, 7])
+def test_contact_virial_between_one_launch_steps(every, prec):
+    w = W.dem_packed_bed(n=900, box=(0.02, 0.02, 0.2), vmax=0.02, seed=3)
+    a, b = _pair(w, prec, 10 * every, lambda s: s.set_virial(every))
+    _same(a, b)
+    ta, tb = a.thermo(energy=True), b.thermo(energy=True)
+    assert ta == tb and any(ta["virial"])
+    a.close()
+    b.close()
