@@ -1203,15 +1203,27 @@ __global__ void __launch_bounds__(256) k_finish_rows(
             nnb[q] = cnt;
             if (nx) nx[q] = xs;  // tile rows: image-owned pairs kept apart
         }
-        if (__ballot(cnt > uint32_t(maxnb)) == 0ull) return;
+        // A context's first build mostly finds nearly every row too long. One word
+        // takes an atomic every 27 ns (three from each wavefront were 5 ms of
+        // the first build of 4,000,000 spheres), so a block sends one, if its
+        // row is longer than what is there, and the first reports the build.
+        __shared__ uint32_t longest[4];
+        uint32_t most = cnt > uint32_t(maxnb) ? cnt : 0u;
+        if (__ballot(most != 0u) != 0ull) {
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            const uint32_t x = __shfl_xor(cnt, o, 64);
-            cnt = x > cnt ? x : cnt;
+            for (int o = 32; o > 0; o >>= 1) {
+                const uint32_t x = __shfl_xor(most, o, 64);
+                most = x > most ? x : most;
+            }
         }
-        if ((threadIdx.x & 63u) == 0u) {
-            atomicMax(&st->max_row, int(cnt));
-            build_failed(st, 2u);
+        if ((threadIdx.x & 63u) == 0u) longest[threadIdx.x >> 6] = most;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            for (int w = 1; w < 4; w++) most = longest[w] > most ? longest[w] : most;
+            if (int(most) > __hip_atomic_load(&st->max_row, __ATOMIC_RELAXED,
+                                              __HIP_MEMORY_SCOPE_AGENT) &&
+                atomicMax(&st->max_row, int(most)) == 0)
+                build_failed(st, 2u);
         }
         return;
     }
