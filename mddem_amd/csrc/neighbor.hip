@@ -721,7 +721,7 @@ __global__ void __launch_bounds__(256) k_build_tiles(CellArgs a) {
 // own test and finds itself in its list, where the entries before it (pairs
 // the other particle owns) end. 256,000 LJ atoms: 117 us (43.2 M vector and
 // 26.6 M scalar instructions) against 165 us (56.5 M and 32.8 M) for rows
-// written entry by entry as they are found; 4,000 atoms 35 against 58 us, the
+// written entry by entry as they are found; 4,000 atoms 18.5 against 58 us, the
 // cells shared by four wavefronts. Issue of the tests bounds it.
 //
 // In a batched ensemble (BATCH) the cell space is shared: the wave finds its
@@ -1747,11 +1747,11 @@ void rebuild_prepare(Ctx& c) {
 // log2 of the wavefronts that share a cell's members in k_build_rows. Each of
 // them reads the cell's candidates, so sharing pays while the cells alone leave
 // the chip's 4096 wavefront places (256 CUs x 16) idle. Whole rebuilds of LJ
-// fluids with 1, 2 and 4 wavefronts per cell, in us: 4,000 atoms (216 cells)
-// 121, 98, 91; 11,000 104, 94, 92; 20,000 (850 cells) 114, 104, 105; 49,000
-// (2,100) 147, 139, 151; 144,000 (6,200) 203, 198, 205; 256,000 (11,000) 263,
-// 261, 284; 500,000 (21,600) 376, 400, 473.
-int build_waves_log2(double cells) { return cells < 896.0 ? 2 : (cells < 10240.0 ? 1 : 0); }
+// fluids with 1, 2 and 4 wavefronts per cell, in us: 4,000 atoms (125 cells in
+// the box) 97, 79, 72; 11,000 (512) 79, 72, 71; 20,000 (1,000) 85, 80, 81;
+// 32,000 (1,331) 98, 91, 93; 49,000 (2,197) 101, 99, 106; 98,000 (4,913) 124,
+// 125, 141; 144,000 (6,859) 147, 150, 173; 256,000 (12,167) 200, 214, 256.
+int build_waves_log2(double cells) { return cells < 896.0 ? 2 : (cells < 3600.0 ? 1 : 0); }
 
 // one build of images, bins and rows with the current capacities; the
 // status says afterwards whether everything fitted
@@ -1875,7 +1875,8 @@ void rebuild_attempt(Ctx& c) {
         // on (490 to 680). With 10, whole rebuilds took 126 us instead of 105
         // at 49,000 atoms, 231 instead of 208 at 256,000. The wider bins of a
         // box of few cells need 16, at 3 wavefronts (4,000 atoms: 5 bins a
-        // side, 860 candidates; from memory their build takes 58 us, not 35).
+        // side, 860 candidates; from memory their whole rebuild takes 93 us,
+        // not 72).
         const double cand = double(n) / c.bins_in_box * double(c.full.size());
         if (c.nsys > 0)
             launch(c, k_build_rows<false, true, 10>, rblocks, 256, ca, wl);
