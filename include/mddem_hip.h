@@ -365,8 +365,8 @@ int mdd_set_lj_positions(mdd_ctx* ctx, int mode);
 int mdd_set_force_lanes(mdd_ctx* ctx, int log2_lanes);
 /* Neighbor-row build kernel: 0 (default) picks by grid occupancy, 1 one
  * wavefront per bin cell, 2 one lane per particle or image (for sparse grids
- * with fewer particles than cells; not used for batched ensembles or LJ cell
- * tiles). Both produce identical rows. No reference counterpart: tuning. */
+ * with fewer particles than cells; not used for LJ cell tiles). Both produce
+ * identical rows. No reference counterpart: tuning. */
 int mdd_set_build_kernel(mdd_ctx* ctx, int mode);
 /* Issue each neighbor rebuild (wrap, spatial sort, images, bins, rows) as one
  * HIP graph launch (default on). The rebuild's launches are recorded with

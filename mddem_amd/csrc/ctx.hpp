@@ -499,7 +499,7 @@ struct Ctx {
     // neighbor build kernel: 0 chosen by occupancy, 1 one wavefront per cell,
     // 2 one lane per member slot (sparse grids)
     int build_mode = 0;
-    DBuf<uint32_t> bin_cell;  // cell of every bin slot (sparse build)
+    DBuf<uint32_t> bin_cell;  // cell of every bin slot (build by members)
     int tile_cap = 0;
     DBuf<uint16_t> crow;
     DBuf<uint32_t> xnbr, nx;

@@ -57,14 +57,16 @@ def test_rows_of_the_others_stay(name, where):
     s.close()
 
 
+@pytest.mark.parametrize("build", [1, 2])
 @pytest.mark.parametrize("where", list(BAD))
-def test_a_bad_system_of_a_batch_leaves_the_rest(where):
+def test_a_bad_system_of_a_batch_leaves_the_rest(where, build):
     ws = [W.gas_system(200 + 50 * k, 0.25, 0.9, 0.4, seed=70 + k) for k in range(3)]
 
     def run(bad):
         s = hip.System(hip.MODEL_DEM, hip.FP64)
         s.set_neighbor(1.1, 0.0, 0, True, 1000, True)
         s.set_dt(ws[0].dt)
+        s.set_build_kernel(build)
         s.set_rebuild_on_box_exit(False)  # an infinite position is outside at every step
         for k, w in enumerate(ws):
             pos = w.pos.copy()
