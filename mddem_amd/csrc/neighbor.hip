@@ -875,10 +875,13 @@ __global__ void __launch_bounds__(256) k_build_rows(CellArgs a, int wpc_log2) {
     const uint32_t pitch = (maxnb + 2u) | 2u;
     // one window, at least one list in LDS and members of one kind (a particle
     // and an image share a cell only where rounding puts an image inside the
-    // box), else each entry goes straight to memory as it is found
+    // box), else each entry goes straight to memory as it is found. So it does
+    // from a list of up to two chunks, for which the lists in LDS are a detour
+    // (whole rebuilds with and without it: gases of 1,000,000 spheres at 1.2 per
+    // cell 1478 / 976 us, at 2.9 894 / 748, at 6 680 / 677, and 713 with up to four chunks)
     const uint32_t np_cell = a.lstart[C + 1] - a.lstart[C];
     const bool images = np_cell == 0u;
-    const bool staged = total <= kWin && pitch <= uint32_t(kStage) &&
+    const bool staged = total > 128u && total <= kWin && pitch <= uint32_t(kStage) &&
                         (images || np_cell == i1 - i0);
     uint32_t cap = staged ? uint32_t(kStage) / pitch : 64u;
     if (cap > 64u) cap = 64u;
@@ -1784,9 +1787,11 @@ void rebuild_attempt(Ctx& c) {
     c.bin_gidx.resize(nall_max);
     // sparse grids (fewer particles than cells): the per-member build kernel.
     // Whole rebuilds of batches, a wavefront per cell / a lane per member, in us:
-    // 64 systems of 600 spheres at 0.16 per cell 353 / 154, at 1.2 181 / 224; 60 of
-    // 12,000 at 0.24 3182 / 386, at 0.77 1590 / 390, at 3.6 704 / 658; 8 of 600 at
-    // 0.15 123 / 107, at 0.47 102 / 118, at 1.2 99 / 170.
+    // 64 systems of 600 spheres at 0.16 per cell 286 / 154, at 1.2 178 / 224; 60 of
+    // 12,000 at 0.09 3384 / 477, at 1.5 818 / 441, at 3.6 681 / 658; 8 of 600 at
+    // 0.15 123 / 107, at 0.47 102 / 118, at 1.2 99 / 170. (Large dilute systems would
+    // gain beyond the line as well, but not where few of their cells hold most of
+    // the particles.)
     const bool sparse = !c.want_tile() &&
                         (c.build_mode == 2 || (c.build_mode == 0 && n < ncells));
     if (sparse) c.bin_cell.resize(nall_max);

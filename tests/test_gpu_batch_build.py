@@ -63,3 +63,22 @@ def test_batch_rows_are_the_same_either_way(kind, bins, prec):
     assert a["rebuilds"] > 1 and (kind == "one" or len(a["owner"]) > 0)
     for k in a:
         assert np.array_equal(a[k], b[k]) and np.array_equal(a[k], c[k]), k
+
+
+@pytest.mark.parametrize("phi", [0.1, 0.17, 0.3])
+def test_rows_around_two_chunks_of_candidates(phi):
+    # cells with about 80, 140 and 240 candidates: up to 128 their rows are written
+    # as they are found, beyond from lists
+    n = 30000
+    w = W.gas_system(n, phi, 0.9, 0.4, seed=8)
+    w.pos = W.Stream(12).uniform(3 * n).reshape(-1, 3) * w.hi  # off its lattice
+    rows = []
+    for mode in (1, 2):
+        s = hip.from_workload(w, hip.MIXED, box_exit=False)
+        s.set_build_kernel(mode)
+        s.bin_neighbor_list()
+        rows.append(s.pairs())
+        s.close()
+    assert len(rows[0][0]) > 0
+    for x, y in zip(*rows):
+        assert np.array_equal(x, y)
