@@ -197,7 +197,7 @@ __device__ inline void image_flags(const BoxP& box, double gc, const double x[3]
 // The last pass of the sort and the first of the images as well: a thread takes
 // a placed element, ranks it inside its cell and moves it there, then counts
 // its periodic images. It moves about 330 B per particle (LJ, mixed), which
-// bounds it: 21 us at 256,000 particles, 8 us at 4,000. As kernels of their own
+// bounds it: 22 us at 256,000 particles, 9 us at 4,000. As kernels of their own
 // move, rank, image count and its scan took 36 us (5 launches) and 19 us (4).
 template <bool PLACED>
 __global__ void __launch_bounds__(256) k_permute(PermArgs a) {
